@@ -281,8 +281,11 @@ int ocu_mg_prolong_bc_ok(const ocu_grid3d *u_coarse, const ocu_grid3d *u_fine,
  * relax(nu2); every level's u (with ghosts) and b (below the top) is written
  * back.  Arrays u[l], b[l], p[l] and h[3l..3l+2] (hx,hy,hz) describe level
  * top+l; zero_top: the top level's u is the zero grid (not read; needs
- * homogeneous faces).  Faces must be Neumann or Dirichlet; the boxes must
- * fit ocu_mg_bottom_lds_bytes() <= ocu_mg_bottom_lds_max(). */
+ * homogeneous faces).  u[0]'s ghost layer holds its level-1 fill, as it does
+ * wherever the solver calls this: with homogeneous faces it is taken from
+ * the cells and not read.  Faces must be Neumann or Dirichlet, or periodic
+ * pairs with even counts; the boxes must fit ocu_mg_bottom_lds_bytes() <=
+ * ocu_mg_bottom_lds_max(). */
 int ocu_mg_bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p,
                          const double *h, int nlev, const ocu_bc_set *bc, int nu1, int nu2,
                          int coarse_iters, int coarse_mode, int zero_top, void *stream);
@@ -298,8 +301,10 @@ size_t ocu_mg_bottom_lds_max(void);
  * mode 1: FP32 grids relaxed in double (copy in, `iterations` host-order
  *   RB-GS iterations with a level-1 ghost fill after every colour, round
  *   back to float) - the coarsest solve of the mixed-precision solver.
- * order: 0 red-black, 1 black-red, 2 symmetric (as relax()).  The grid must
- * fit in 64 KiB of LDS (u and b in the compute type, ghosts included). */
+ * order: 0 red-black, 1 black-red, 2 symmetric (as relax()).  u's ghost layer
+ * holds its fill, as it does wherever the solver calls this: with
+ * homogeneous faces it is taken from the cells and not read.  A grid beyond
+ * one workgroup's LDS is relaxed in global memory. */
 int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
                         const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy,
                         double hz, int mode, void *stream);

@@ -1848,6 +1848,691 @@ __global__ __launch_bounds__(BOT_THREADS) void k_mg_bottom(BotArgs<T, TC> args) 
   }
 }
 
+// ------------------------------------------------------------------------
+// division by a diagonal known in advance
+// ------------------------------------------------------------------------
+//
+// The relaxation divides by the diagonal, of which a level has 27 values
+// (none, low or high face per axis).  An IEEE division is about 11 VALU
+// instructions in FP32 and 14 in FP64 with a quarter-rate reciprocal in its
+// dependency chain; with the divisor's reciprocal at hand the same quotient,
+// bit for bit, takes 3 and 6:
+//   FP32: x times the double nearest 1/d, rounded once to float.  The double
+//     product is within 2^-52 (relative) of x/d, and a quotient of two floats
+//     keeps 2^-49 away from the middle between two floats (x = m*d with a
+//     25-bit odd m would need 25 bits in x), so the rounding is the
+//     quotient's; zeros, infinities and NaN come out as in a division, and a
+//     quotient below 2^-126 may end one denormal unit (1.4e-45) away.
+//   FP64: two fused corrections of x*r.  The first leaves a faithful
+//     quotient, whose remainder is exact, and by Markstein's theorem the
+//     second then rounds correctly, r being the correctly rounded 1/d;
+//     div_fixup gives the special operands their IEEE results.  (|x| below
+//     2^-960 would make the remainder inexact: one unit of a 1e-290 value.)
+template <typename T> struct Recip;
+template <> struct Recip<float> {
+  double r;
+};
+template <> struct Recip<double> {
+  double d, r;
+};
+__device__ __forceinline__ Recip<float> recip_of(float d) { return {1.0 / (double)d}; }
+__device__ __forceinline__ Recip<double> recip_of(double d) { return {d, 1.0 / d}; }
+__device__ __forceinline__ float div_by(float x, const Recip<float> &q) { return (float)((double)x * q.r); }
+__device__ __forceinline__ double div_by(double x, const Recip<double> &q) {
+  double y = x * q.r;
+  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
+  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
+  return __builtin_amdgcn_div_fixup(y, q.d, x);
+}
+
+// ------------------------------------------------------------------------
+// the bottom of a V-cycle, a thread per coarse cell
+// ------------------------------------------------------------------------
+//
+// The same work as k_mg_bottom (which keeps the rest: inhomogeneous faces,
+// levels that are not exactly halved, unaligned rows) for the hierarchies
+// the solvers make: every
+// level exactly twice the next one, homogeneous faces, and u's ghost layer
+// the level-1 fill of u.  One workgroup on one CU is bound by its issue slots
+// (16^3: 2048 cells per colour on four SIMDs) and, on the small levels, by
+// the latency of one cell's chain; so:
+//   - a thread owns a block of 2x2x2 cells, the children of one coarse cell.
+//     A colour is four cells of the block, each with three neighbours in the
+//     thread's registers and three in LDS, and four independent chains to
+//     hide latency; residual + restriction are local to the thread, and one
+//     27-cell neighbourhood prolongs to all eight cells.
+//   - no ghost cells: a ghost is its source cell's value (Neumann), that
+//     with the sign changed (Dirichlet, SIGN) or the cell at the other end
+//     (periodic), so a face neighbour is an address chosen once per level,
+//     and nothing is stored or branched on at the boundary.
+//   - LDS holds a block's eight cells with a stride of nine: consecutive
+//     threads fall on different banks and a neighbour's cell is an
+//     immediate offset.
+//   - the diagonals' reciprocals come from a 27-entry table (Recip).
+//   - a level of at most 64 blocks (8^3), or a coarsest level of at most 64
+//     cell pairs, is one wave's work: LDS operations of a wave are ordered, so
+//     it needs no barriers between colours.
+// Measured against k_mg_bottom (one launch, launches included): 16^3 down to
+// 4^3 46.1 -> 21.6 us in FP64, 39.0 -> 18.3 mixed, 37.4 -> 17.7 in FP32;
+// 24x20x28 over 12x10x14 (84 coarsest iterations) in FP32 165 -> 62 us; the
+// coarsest level by itself (k_coarse_pairs against k_coarse) 22.4 -> 7.1 us
+// at 4^3 and 592 -> 43 us at 12x10x14.
+// The coarsest level (odd sizes allowed) gives a thread one pair of cells
+// (k even, k odd), one of each colour, with the two colours in arrays of
+// their own, so both colours' reads are unit stride.
+constexpr int BLK = 9;
+constexpr int FACE_CLASSES = 27;
+
+struct PairGeom {
+  int nx, ny, nz, npz, n;  // cells; pairs along k and in all
+  Mag my, mz, mpy, mpz, mpair;  // ny, nz, ny+2, nz+2, npz
+};
+
+template <typename T>
+struct BlkLevel {
+  DGrid<T> u, b;
+  int bx, by, bz, nb;  // blocks
+  Mag mby, mbz, mpy, mpz, my, mz;  // by, bz, ny+2, nz+2, ny, nz
+  int uoff, boff, toff;            // LDS byte offsets: u, b, reciprocals
+  typename DevCFor<T>::type dc;
+  ResC<T> rc;
+};
+
+template <typename T, typename TC>
+struct BlkArgs {
+  BlkLevel<T> L[BOT_MAX - 1];  // the levels above the coarsest
+  DGrid<T> cu, cb;             // the coarsest
+  PairGeom cg;
+  int cuoff, cboff, ctoff;
+  HostC<TC> hc;
+  int per[3];
+  unsigned flip;  // bit f: face f (x high, x low, y high, ...) is Dirichlet
+  int nlev, nu1, nu2, zero_top, coarse_iters, pow2;
+};
+static_assert(sizeof(BlkArgs<double, double>) <= 4096 && sizeof(BlkArgs<float, double>) <= 4096,
+              "bottom launch arguments exceed the kernel argument segment");
+
+__device__ __forceinline__ float flip_sign(float v, int m) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, v) ^ m);
+}
+__device__ __forceinline__ double flip_sign(double v, int m) {
+  return __builtin_bit_cast(double, __builtin_bit_cast(long long, v) ^ ((long long)m << 32));
+}
+
+// order LDS accesses between the lanes of one wave (executed in order) or,
+// through the barrier, between the waves of the block
+__device__ __forceinline__ void lds_sync(bool one_wave) {
+  if (one_wave) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
+// the diagonals of a level: class of an axis 0 none, 1 low face, 2 high
+// face; the additions in diag_dev's and diag_host's order
+__device__ __forceinline__ int face_class(bool lo, bool hi) { return lo ? 1 : hi ? 2 : 0; }
+template <typename T, typename C>
+__device__ __forceinline__ Recip<T> class_recip(const C &c, int q) {
+  const int x = q / 9, y = (q / 3) % 3, z = q % 3;
+  T d = c.ld;
+  if (x) d += c.m[x == 2 ? 0 : 1];
+  if (y) d += c.m[y == 2 ? 2 : 3];
+  if (z) d += c.m[z == 2 ? 4 : 5];
+  return recip_of(d);
+}
+
+// relax_pt with b's term and the diagonal's reciprocal in hand
+__device__ __forceinline__ double b_term(const DevC64 &c, double b) { return c.neg_hsq * b; }
+__device__ __forceinline__ float b_term(const DevC32 &c, float b) { return -c.hsq * b; }
+__device__ __forceinline__ double relax_pt_q(const DevC64 &c, double uc, double zm, double zp, double ym, double yp,
+                                             double xm, double xp, double hb, const Recip<double> &q) {
+  double r = -c.ld * uc;
+  r += c.fz * (zm + zp);
+  r += c.fy * (ym + yp);
+  r += c.fx * (xm + xp);
+  r += hb;
+  return uc + div_by(c.omega * r, q);
+}
+__device__ __forceinline__ float relax_pt_q(const DevC32 &c, float uc, float zm, float zp, float ym, float yp,
+                                            float xm, float xp, float hb, const Recip<float> &q) {
+  float r = (hb - c.ld * uc);
+  r += c.fz * (zm + zp);
+  r += c.fy * (ym + yp);
+  r += c.fx * (xm + xp);
+  return uc + div_by(c.omega * r, q);
+}
+
+// a thread's block of a level: its cells (e = 4*dx + 2*dy + dz), b's terms,
+// reciprocals, and the LDS element of the first cell across each face (x
+// high, x low, ...: the block's own where the ghost derives from it) with
+// the sign change of a Dirichlet ghost
+template <typename T>
+struct Blk {
+  T u[8], hb[8];
+  Recip<T> q[8];
+  int own, a[6], m[6];
+};
+
+template <typename T>
+__device__ __forceinline__ void blk_coords(const BlkLevel<T> &L, int blk, int &ic, int &jc, int &kc) {
+  const int row = mdiv(blk, L.mbz);
+  kc = blk - row * L.bz;
+  ic = mdiv(row, L.mby);
+  jc = row - ic * L.by;
+}
+
+template <bool SIGN, typename T>
+__device__ __forceinline__ void blk_faces(Blk<T> &s, const BlkLevel<T> &L, const int *per, unsigned flip, int blk,
+                                          int ic, int jc, int kc) {
+  const int c[3] = {ic, jc, kc}, n[3] = {L.bx, L.by, L.bz}, st[3] = {L.by * L.bz, L.bz, 1}, ch[3] = {4, 2, 1};
+  s.own = blk * BLK;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const bool hi = c[a] == n[a] - 1, lo = c[a] == 0;
+    const int wrap = (n[a] - 1) * st[a];
+    s.a[2 * a] = !hi ? (blk + st[a]) * BLK : per[a] ? (blk - wrap) * BLK : s.own + ch[a];
+    s.a[2 * a + 1] = !lo ? (blk - st[a]) * BLK + ch[a] : per[a] ? (blk + wrap) * BLK + ch[a] : s.own;
+    if (SIGN) {
+      s.m[2 * a] = hi && ((flip >> (2 * a)) & 1) ? (int)0x80000000 : 0;
+      s.m[2 * a + 1] = lo && ((flip >> (2 * a + 1)) & 1) ? (int)0x80000000 : 0;
+    }
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void blk_recips(Blk<T> &s, const BlkLevel<T> &L, const Recip<T> *tab, int ic, int jc,
+                                           int kc) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const int x = (e & 4) ? (ic == L.bx - 1 ? 2 : 0) : (ic == 0 ? 1 : 0);
+    const int y = (e & 2) ? (jc == L.by - 1 ? 2 : 0) : (jc == 0 ? 1 : 0);
+    const int z = (e & 1) ? (kc == L.bz - 1 ? 2 : 0) : (kc == 0 ? 1 : 0);
+    s.q[e] = tab[(x * 3 + y) * 3 + z];
+  }
+}
+
+// the six neighbours of cell e of a block
+template <bool SIGN, typename T>
+__device__ __forceinline__ void blk_nbrs(const Blk<T> &s, const T *U, int e, T &zm, T &zp, T &ym, T &yp, T &xm,
+                                         T &xp) {
+  auto out = [&](int f, int in_plane) {
+    T v = U[s.a[f] + in_plane];
+    return SIGN ? flip_sign(v, s.m[f]) : v;
+  };
+  const int dx = e >> 2, dy = (e >> 1) & 1, dz = e & 1;
+  zm = dz ? s.u[e ^ 1] : out(5, e & 6);
+  zp = dz ? out(4, e & 6) : s.u[e ^ 1];
+  ym = dy ? s.u[e ^ 2] : out(3, e & 5);
+  yp = dy ? out(2, e & 5) : s.u[e ^ 2];
+  xm = dx ? s.u[e ^ 4] : out(1, e & 3);
+  xp = dx ? out(0, e & 3) : s.u[e ^ 4];
+}
+
+template <bool SIGN, int COL, typename T, typename C>
+__device__ __forceinline__ void blk_colour(Blk<T> &s, T *U, const C &c) {
+  constexpr int cells[2][4] = {{0, 3, 5, 6}, {1, 2, 4, 7}};
+  T v[4];
+#pragma unroll
+  for (int n = 0; n < 4; n++) {
+    const int e = cells[COL][n];
+    T zm, zp, ym, yp, xm, xp;
+    blk_nbrs<SIGN>(s, U, e, zm, zp, ym, yp, xm, xp);
+    v[n] = relax_pt_q(c, s.u[e], zm, zp, ym, yp, xm, xp, s.hb[e], s.q[e]);
+  }
+#pragma unroll
+  for (int n = 0; n < 4; n++) U[s.own + cells[COL][n]] = s.u[cells[COL][n]] = v[n];
+}
+
+template <bool SIGN, typename T>
+__device__ __forceinline__ void blk_get(Blk<T> &s, const BlkLevel<T> &L, const int *per, unsigned flip, const T *U,
+                                        const T *B, const Recip<T> *tab, int blk) {
+  int ic, jc, kc;
+  blk_coords(L, blk, ic, jc, kc);
+  blk_faces<SIGN>(s, L, per, flip, blk, ic, jc, kc);
+  blk_recips(s, L, tab, ic, jc, kc);
+#pragma unroll
+  for (int e = 0; e < 8; e++) s.u[e] = U[s.own + e];
+#pragma unroll
+  for (int e = 0; e < 8; e++) s.hb[e] = b_term(L.dc, B[s.own + e]);
+}
+
+// iters red-black iterations; HELD: each thread's only block stays in s
+// (threads past the last block idle), else the blocks are reloaded for
+// every colour.  Ends with the block's threads in step.
+template <bool SIGN, bool HELD, typename T>
+__device__ __forceinline__ void blk_sweeps(Blk<T> &s, const BlkLevel<T> &L, const int *per, unsigned flip, T *U,
+                                           const T *B, const Recip<T> *tab, int iters) {
+  const typename DevCFor<T>::type c = L.dc;
+  if (HELD) {
+    const bool one = L.nb <= 64, mine = (int)threadIdx.x < L.nb;
+    for (int it = 0; it < iters; it++) {
+      if (mine) blk_colour<SIGN, 0>(s, U, c);
+      lds_sync(one);
+      if (mine) blk_colour<SIGN, 1>(s, U, c);
+      lds_sync(one);
+    }
+    if (one) __syncthreads();
+  } else {
+    for (int it = 0; it < iters; it++) {
+      for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+        blk_get<SIGN>(s, L, per, flip, U, B, tab, blk);
+        blk_colour<SIGN, 0>(s, U, c);
+      }
+      __syncthreads();
+      for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+        blk_get<SIGN>(s, L, per, flip, U, B, tab, blk);
+        blk_colour<SIGN, 1>(s, U, c);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// residuals of a block's cells and their restriction (res_val, restrict_sum)
+template <bool SIGN, typename T>
+__device__ __forceinline__ T blk_restrict(const Blk<T> &s, const T *U, const T *B, const ResC<T> &c) {
+  T r[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    T zm, zp, ym, yp, xm, xp;
+    blk_nbrs<SIGN>(s, U, e, zm, zp, ym, yp, xm, xp);
+    r[e] = res_val(c, B[s.own + e], zm, zp, ym, yp, xm, xp, s.u[e]);
+  }
+  return restrict_sum(r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]);
+}
+
+// LDS element of cell (i,j,k): block layout, and the coarsest's pairs
+template <typename T>
+__device__ __forceinline__ int blk_elem(const BlkLevel<T> &L, int i, int j, int k) {
+  return (((i >> 1) * L.by + (j >> 1)) * L.bz + (k >> 1)) * BLK + 4 * (i & 1) + 2 * (j & 1) + (k & 1);
+}
+__device__ __forceinline__ int pair_elem(const PairGeom &g, int i, int j, int k) {
+  return ((i + j + k) & 1) * g.n + (i * g.ny + j) * g.npz + (k >> 1);
+}
+
+// the 27 cells around coarse cell (ic,jc,kc), ghosts as the level-1 fill
+// has them (x, y and z sign changes commute), read through `at`
+template <bool SIGN, typename T, typename AT>
+__device__ __forceinline__ void coarse_around(T (&v)[3][3][3], int ic, int jc, int kc, int nx, int ny, int nz,
+                                              const int *per, unsigned flip, AT at) {
+  const int c[3] = {ic, jc, kc}, n[3] = {nx, ny, nz};
+  int ix[3][3], m[3][3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const bool lo = c[a] == 0, hi = c[a] == n[a] - 1;
+    ix[a][0] = !lo ? c[a] - 1 : per[a] ? n[a] - 1 : 0;
+    ix[a][1] = c[a];
+    ix[a][2] = !hi ? c[a] + 1 : per[a] ? 0 : n[a] - 1;
+    m[a][0] = lo && ((flip >> (2 * a + 1)) & 1) ? (int)0x80000000 : 0;
+    m[a][1] = 0;
+    m[a][2] = hi && ((flip >> (2 * a)) & 1) ? (int)0x80000000 : 0;
+  }
+#pragma unroll
+  for (int x = 0; x < 3; x++)
+#pragma unroll
+    for (int y = 0; y < 3; y++)
+#pragma unroll
+      for (int z = 0; z < 3; z++) {
+        const T t = at(ix[0][x], ix[1][y], ix[2][z]);
+        v[x][y][z] = SIGN ? flip_sign(t, m[0][x] ^ m[1][y] ^ m[2][z]) : t;
+      }
+}
+
+// the prolongation into a block's eight cells (k_prolong's operations and
+// corner choice)
+template <typename T>
+__device__ __forceinline__ void blk_prolong(T (&u)[8], const T (&v)[3][3][3]) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const int dx = e >> 2, dy = (e >> 1) & 1, dz = e & 1, x = 2 * dx, y = 2 * dy, z = 2 * dz;
+    const int cx = (dx == 0 && dy == 1 && dz == 1) ? 2 : x;
+    u[e] = u[e] + PW<T>::c0 * v[1][1][1] + PW<T>::c1 * (v[x][1][1] + v[1][y][1] + v[1][1][z]) +
+           PW<T>::c2 * (v[x][y][1] + v[x][1][z] + v[1][y][z]) + PW<T>::c3 * v[cx][y][z];
+  }
+}
+
+// the ghost layer of a finished level to global memory: edges and corners
+// too, each from the cell it derives from, read through `at`
+template <bool SIGN, typename T, typename AT>
+__device__ __forceinline__ void shell_store(const DGrid<T> &o, Mag mpy, Mag mz, const int *per, unsigned flip, AT at) {
+  const int nx = o.nx, ny = o.ny, nz = o.nz;
+  const int nZ = (nx + 2) * (ny + 2), nY = (nx + 2) * nz, nX = ny * nz;
+  for (int t = threadIdx.x; t < 2 * (nZ + nY + nX); t += blockDim.x) {
+    int i, j, k, q = t;
+    if (q < 2 * nZ) {
+      const int side = q >= nZ;
+      q -= side * nZ;
+      i = mdiv(q, mpy);
+      j = q - i * (ny + 2) - 1;
+      i -= 1;
+      k = side ? nz : -1;
+    } else if ((q -= 2 * nZ) < 2 * nY) {
+      const int side = q >= nY;
+      q -= side * nY;
+      i = mdiv(q, mz);
+      k = q - i * nz;
+      i -= 1;
+      j = side ? ny : -1;
+    } else {
+      q -= 2 * nY;
+      const int side = q >= nX;
+      q -= side * nX;
+      j = mdiv(q, mz);
+      k = q - j * nz;
+      i = side ? nx : -1;
+    }
+    const int c[3] = {i, j, k}, n[3] = {nx, ny, nz};
+    int s[3], m = 0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const bool lo = c[a] < 0, hi = c[a] >= n[a];
+      s[a] = lo ? (per[a] ? n[a] - 1 : 0) : hi ? (per[a] ? 0 : n[a] - 1) : c[a];
+      if (SIGN) m ^= (lo && ((flip >> (2 * a + 1)) & 1)) || (hi && ((flip >> (2 * a)) & 1)) ? (int)0x80000000 : 0;
+    }
+    const T v = at(s[0], s[1], s[2]);
+    o.at(i, j, k) = SIGN ? flip_sign(v, m) : v;
+  }
+}
+
+// ---- the coarsest level: relax_on_host arithmetic on pairs of cells ----
+
+// one cell of a thread's pair: its LDS element, its neighbours' (z low, z
+// high, y low, y high, x low, x high) and their ghosts' sign changes
+template <typename T>
+struct PairCell {
+  T u, hb;
+  Recip<T> q;
+  int own, a[6], m[6];
+  bool in;
+};
+
+template <bool SIGN, typename T>
+__device__ __forceinline__ void pair_cell(PairCell<T> &s, const PairGeom &g, const int *per, unsigned flip,
+                                          const Recip<T> *tab, int col, int p) {
+  const int row = mdiv(p, g.mpair), m = p - row * g.npz, i = mdiv(row, g.my), j = row - i * g.ny;
+  const int e = (i + j + col) & 1, k = 2 * m + e;
+  s.in = p < g.n && k < g.nz;
+  s.own = col * g.n + p;
+  const int oth = (1 - col) * g.n + p, sx = g.ny * g.npz, sy = g.npz;
+  s.a[0] = k > 0 ? (e ? oth : oth - 1) : per[2] ? oth + g.npz - 1 : s.own;
+  s.a[1] = k < g.nz - 1 ? (e ? oth + 1 : oth) : per[2] ? oth - (g.npz - 1) : s.own;
+  s.a[2] = j > 0 ? oth - sy : per[1] ? oth + (g.ny - 1) * sy : s.own;
+  s.a[3] = j < g.ny - 1 ? oth + sy : per[1] ? oth - (g.ny - 1) * sy : s.own;
+  s.a[4] = i > 0 ? oth - sx : per[0] ? oth + (g.nx - 1) * sx : s.own;
+  s.a[5] = i < g.nx - 1 ? oth + sx : per[0] ? oth - (g.nx - 1) * sx : s.own;
+  if (SIGN) {
+    const bool at[6] = {k == 0, k == g.nz - 1, j == 0, j == g.ny - 1, i == 0, i == g.nx - 1};
+    const int f[6] = {5, 4, 3, 2, 1, 0};
+#pragma unroll
+    for (int n = 0; n < 6; n++) s.m[n] = at[n] && ((flip >> f[n]) & 1) ? (int)0x80000000 : 0;
+  }
+  s.q = tab[(face_class(i == 0, i == g.nx - 1) * 3 + face_class(j == 0, j == g.ny - 1)) * 3 +
+            face_class(k == 0, k == g.nz - 1)];
+}
+
+// do_cpu_solve's update with b's term in hand.  P2: T is float and the
+// three factors are powers of two, so a product with one is exact and the
+// float sum of two floats is what rounding their double sum gives (double
+// keeps more than twice float's bits); the sums stay in float then.
+template <bool P2, typename T>
+__device__ __forceinline__ T relax_host_q(const HostC<T> &c, T uc, T zm, T zp, T ym, T yp, T xm, T xp, T hb,
+                                          const Recip<T> &q) {
+  T r = (hb - c.ld * uc);
+  if (P2) {
+    r += (T)c.fz * (zm + zp);
+    r += (T)c.fy * (yp + ym);
+    r += (T)c.fx * (xp + xm);
+  } else {
+    r += c.fz * (zm + zp);
+    r += c.fy * (yp + ym);
+    r += c.fx * (xp + xm);
+  }
+  return uc + div_by(c.omega * r, q);
+}
+
+template <bool SIGN, bool P2, typename T>
+__device__ __forceinline__ void pair_relax(PairCell<T> &s, T *U, const HostC<T> &c) {
+  T v[6];
+#pragma unroll
+  for (int n = 0; n < 6; n++) {
+    v[n] = U[s.a[n]];
+    if (SIGN) v[n] = flip_sign(v[n], s.m[n]);
+  }
+  s.u = relax_host_q<P2>(c, s.u, v[0], v[1], v[2], v[3], v[4], v[5], s.hb, s.q);
+  U[s.own] = s.u;
+}
+
+// `iterations` iterations of relax_on_host on U (b in B), colours in
+// `order`'s sequence.  At most one pair per thread: both cells stay in
+// registers, and up to 64 pairs are one wave's work without barriers.  Ends
+// with the block's threads in step.
+template <bool SIGN, bool P2, typename T>
+__device__ __forceinline__ void pair_sweeps(T *U, const T *B, const PairGeom &g, const HostC<T> &cc, const int *per,
+                                            unsigned flip, const Recip<T> *tab, int iterations, int order) {
+  const HostC<T> c = cc;
+  auto fill = [&](PairCell<T> &s, int col, int p) {
+    pair_cell<SIGN>(s, g, per, flip, tab, col, p);
+    if (s.in) {
+      s.u = U[s.own];
+      s.hb = -c.h * c.h * B[s.own];
+    }
+  };
+  if (g.n <= (int)blockDim.x) {
+    const bool one = g.n <= 64;
+    if (!one || threadIdx.x < 64) {
+      PairCell<T> s[2];
+      fill(s[0], 0, threadIdx.x);
+      fill(s[1], 1, threadIdx.x);
+      for (int it = 0; it < iterations; it++) {
+        // uniform: the second half of the symmetric order starts black
+        if (color_of(order, it, iterations, 0) == 0) {
+          if (s[0].in) pair_relax<SIGN, P2>(s[0], U, c);
+          lds_sync(one);
+          if (s[1].in) pair_relax<SIGN, P2>(s[1], U, c);
+        } else {
+          if (s[1].in) pair_relax<SIGN, P2>(s[1], U, c);
+          lds_sync(one);
+          if (s[0].in) pair_relax<SIGN, P2>(s[0], U, c);
+        }
+        lds_sync(one);
+      }
+    }
+    if (one) __syncthreads();
+  } else {
+    for (int it = 0; it < iterations; it++)
+      for (int rb = 0; rb < 2; rb++) {
+        const int col = color_of(order, it, iterations, rb);
+        for (int p = threadIdx.x; p < g.n; p += blockDim.x) {
+          PairCell<T> s;
+          fill(s, col, p);
+          if (s.in) pair_relax<SIGN, P2>(s, U, c);
+        }
+        __syncthreads();
+      }
+  }
+}
+template <bool SIGN, typename T>
+__device__ __forceinline__ void pair_solve(T *U, const T *B, const PairGeom &g, const HostC<T> &c, const int *per,
+                                           unsigned flip, const Recip<T> *tab, int iterations, int order, int pow2) {
+  if (sizeof(T) == 4 && pow2) pair_sweeps<SIGN, true>(U, B, g, c, per, flip, tab, iterations, order);
+  else pair_sweeps<SIGN, false>(U, B, g, c, per, flip, tab, iterations, order);
+}
+
+// a finished coarsest level to global memory, ghosts included
+template <bool SIGN, typename TS, typename TC>
+__device__ __forceinline__ void pair_store(const DGrid<TS> &o, const TC *U, const PairGeom &g, const int *per,
+                                           unsigned flip) {
+  auto at = [&](int i, int j, int k) { return (TS)U[pair_elem(g, i, j, k)]; };
+  for (int t = threadIdx.x; t < g.nx * g.ny * g.nz; t += blockDim.x) {
+    const int row = mdiv(t, g.mz), i = mdiv(row, g.my), j = row - i * g.ny, k = t - row * g.nz;
+    o.at(i, j, k) = at(i, j, k);
+  }
+  shell_store<SIGN>(o, g.mpy, g.mz, per, flip, at);
+}
+
+template <typename T>
+struct alignas(2 * sizeof(T)) Two {
+  T a, b;
+};
+
+template <typename T, typename TC, bool SIGN, int MAXT>
+__global__ __launch_bounds__(MAXT) void k_mg_bottom_blocks(BlkArgs<T, TC> args) {
+  // read in place, in the kernel-argument segment (see k_mg_bottom)
+  (void)args;
+  const BlkArgs<T, TC> &A = *(const BlkArgs<T, TC> *)__builtin_amdgcn_kernarg_segment_ptr();
+  extern __shared__ unsigned char smem[];
+  const int C = A.nlev - 1;
+  const int per[3] = {A.per[0], A.per[1], A.per[2]};
+  const unsigned flip = A.flip;
+  auto U = [&](int l) { return (T *)(smem + A.L[l].uoff); };
+  auto B = [&](int l) { return (T *)(smem + A.L[l].boff); };
+  auto tab = [&](int l) { return (const Recip<T> *)(smem + A.L[l].toff); };
+  TC *const uc = (TC *)(smem + A.cuoff), *const bc = (TC *)(smem + A.cboff);
+  const Recip<TC> *const ctab = (const Recip<TC> *)(smem + A.ctoff);
+
+  // the top level's cells, every global load of a block in flight at once
+  {
+    const BlkLevel<T> &L = A.L[0];
+    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+      int ic, jc, kc;
+      blk_coords(L, blk, ic, jc, kc);
+      Two<T> ru[4], rb[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int64_t o = (int64_t)(2 * ic + (q >> 1)), oj = 2 * jc + (q & 1);
+        rb[q] = *reinterpret_cast<const Two<T> *>(L.b.p + o * L.b.xs + oj * L.b.ys + 2 * kc);
+        if (A.zero_top) ru[q] = Two<T>{(T)0, (T)0};
+        else ru[q] = *reinterpret_cast<const Two<T> *>(L.u.p + o * L.u.xs + oj * L.u.ys + 2 * kc);
+      }
+      T *u = U(0) + blk * BLK, *b = B(0) + blk * BLK;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        u[2 * q] = ru[q].a;
+        u[2 * q + 1] = ru[q].b;
+        b[2 * q] = rb[q].a;
+        b[2 * q + 1] = rb[q].b;
+      }
+    }
+  }
+  for (int q = threadIdx.x; q < FACE_CLASSES * A.nlev; q += blockDim.x) {
+    const int l = q / FACE_CLASSES, n = q - l * FACE_CLASSES;
+    if (l < C) ((Recip<T> *)(smem + A.L[l].toff))[n] = class_recip<T>(A.L[l].dc, n);
+    else ((Recip<TC> *)(smem + A.ctoff))[n] = class_recip<TC>(A.hc, n);
+  }
+  __syncthreads();
+
+  // down: relax, residual -> the next level's b; the next u starts at zero
+  for (int l = 0; l < C; l++) {
+    const BlkLevel<T> &L = A.L[l];
+    T *const u = U(l), *const b = B(l);
+    auto to_coarse = [&](const Blk<T> &s, int blk) {
+      int ic, jc, kc;
+      blk_coords(L, blk, ic, jc, kc);
+      const T v = blk_restrict<SIGN>(s, u, b, L.rc);
+      if (l + 1 < C) {
+        const int e = blk_elem(A.L[l + 1], ic, jc, kc);
+        B(l + 1)[e] = v;
+        U(l + 1)[e] = (T)0;
+        A.L[l + 1].b.at(ic, jc, kc) = v;
+      } else {
+        const int e = pair_elem(A.cg, ic, jc, kc);
+        bc[e] = (TC)v;
+        uc[e] = (TC)0;
+        A.cb.at(ic, jc, kc) = v;
+      }
+    };
+    Blk<T> s;
+    if (L.nb <= (int)blockDim.x) {
+      const bool mine = (int)threadIdx.x < L.nb;
+      if (mine) blk_get<SIGN>(s, L, per, flip, u, b, tab(l), threadIdx.x);
+      blk_sweeps<SIGN, true>(s, L, per, flip, u, b, tab(l), A.nu1);
+      if (mine) to_coarse(s, threadIdx.x);
+    } else {
+      blk_sweeps<SIGN, false>(s, L, per, flip, u, b, tab(l), A.nu1);
+      for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+        blk_get<SIGN>(s, L, per, flip, u, b, tab(l), blk);
+        to_coarse(s, blk);
+      }
+    }
+    __syncthreads();
+  }
+
+  pair_solve<SIGN>(uc, bc, A.cg, A.hc, per, flip, ctab, A.coarse_iters, 0, A.pow2);
+  pair_store<SIGN>(A.cu, uc, A.cg, per, flip);
+
+  // up: prolongation, relax, and the finished level to global memory
+  for (int l = C - 1; l >= 0; l--) {
+    const BlkLevel<T> &L = A.L[l];
+    T *const u = U(l), *const b = B(l);
+    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+      int ic, jc, kc;
+      blk_coords(L, blk, ic, jc, kc);
+      T v[3][3][3], w[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) w[e] = u[blk * BLK + e];
+      if (l + 1 < C) {
+        const BlkLevel<T> &N = A.L[l + 1];
+        const T *const un = U(l + 1);
+        coarse_around<SIGN>(v, ic, jc, kc, L.bx, L.by, L.bz, per, flip,
+                            [&](int i, int j, int k) { return un[blk_elem(N, i, j, k)]; });
+      } else {
+        coarse_around<SIGN>(v, ic, jc, kc, L.bx, L.by, L.bz, per, flip,
+                            [&](int i, int j, int k) { return (T)uc[pair_elem(A.cg, i, j, k)]; });
+      }
+      blk_prolong(w, v);
+#pragma unroll
+      for (int e = 0; e < 8; e++) u[blk * BLK + e] = w[e];
+    }
+    __syncthreads();
+    Blk<T> s;
+    if (L.nb <= (int)blockDim.x) {
+      if ((int)threadIdx.x < L.nb) blk_get<SIGN>(s, L, per, flip, u, b, tab(l), threadIdx.x);
+      blk_sweeps<SIGN, true>(s, L, per, flip, u, b, tab(l), A.nu2);
+    } else {
+      blk_sweeps<SIGN, false>(s, L, per, flip, u, b, tab(l), A.nu2);
+    }
+    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+      int ic, jc, kc;
+      blk_coords(L, blk, ic, jc, kc);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        *reinterpret_cast<Two<T> *>(L.u.p + (int64_t)(2 * ic + (q >> 1)) * L.u.xs + (2 * jc + (q & 1)) * L.u.ys +
+                                    2 * kc) = Two<T>{u[blk * BLK + 2 * q], u[blk * BLK + 2 * q + 1]};
+    }
+    shell_store<SIGN>(L.u, L.mpy, L.mz, per, flip, [&](int i, int j, int k) { return u[blk_elem(L, i, j, k)]; });
+  }
+}
+
+// ocu_mg_coarse_relax on pairs: a level by itself, any sizes
+template <typename TS, typename TC>
+struct PairArgs {
+  DGrid<TS> u, b;
+  PairGeom g;
+  HostC<TC> c;
+  int per[3];
+  unsigned flip;
+  int iterations, order, pow2;
+};
+template <typename TS, typename TC, bool SIGN>
+__global__ __launch_bounds__(BOT_THREADS) void k_coarse_pairs(PairArgs<TS, TC> A) {
+  extern __shared__ unsigned char smem[];
+  Recip<TC> *tab = (Recip<TC> *)smem;
+  TC *uc = (TC *)(smem + FACE_CLASSES * sizeof(Recip<double>)), *bc = uc + 2 * A.g.n;
+  for (int t = threadIdx.x; t < A.g.nx * A.g.ny * A.g.nz; t += blockDim.x) {
+    const int row = mdiv(t, A.g.mz), i = mdiv(row, A.g.my), j = row - i * A.g.ny, k = t - row * A.g.nz;
+    const int e = pair_elem(A.g, i, j, k);
+    uc[e] = (TC)A.u.at(i, j, k);
+    bc[e] = (TC)A.b.at(i, j, k);
+  }
+  for (int q = threadIdx.x; q < FACE_CLASSES; q += blockDim.x) tab[q] = class_recip<TC>(A.c, q);
+  __syncthreads();
+  pair_solve<SIGN>(uc, bc, A.g, A.c, A.per, A.flip, tab, A.iterations, A.order, A.pow2);
+  pair_store<SIGN>(A.u, uc, A.g, A.per, A.flip);
+}
+
 FacesS faces_s(const ocu_bc_set *bc) {
   FacesS F;
   const ocu_bc *all[6] = {&bc->xpos, &bc->xneg, &bc->ypos, &bc->yneg, &bc->zpos, &bc->zneg};
@@ -2210,9 +2895,116 @@ size_t bottom_layout(const ocu_grid3d *u, int nlev, int mode, BotArgs<T, TC> *A)
 // single workgroup)
 constexpr size_t BOT_LDS_MAX = 163840;
 
+// homogeneous faces (periodic pairs, or Neumann / Dirichlet with value 0)
+// and even counts along periodic axes: what the block and pair kernels take
+bool plain_faces(const ocu_bc_set *bc, const ocu_grid3d *u, int nlev) {
+  if (!gfaces_paired(bc)) return false;
+  const ocu_bc *all[6] = {&bc->xpos, &bc->xneg, &bc->ypos, &bc->yneg, &bc->zpos, &bc->zneg};
+  for (int f = 0; f < 6; f++)
+    if (all[f]->type != OCU_BC_PERIODIC && all[f]->value != 0.0f) return false;
+  for (int l = 0; l < nlev; l++) {
+    const int n[3] = {u[l].nx, u[l].ny, u[l].nz};
+    for (int a = 0; a < 3; a++)
+      if (all[2 * a]->type == OCU_BC_PERIODIC && n[a] % 2) return false;
+  }
+  return true;
+}
+unsigned dirichlet_faces(const ocu_bc_set *bc) {
+  const ocu_bc *all[6] = {&bc->xpos, &bc->xneg, &bc->ypos, &bc->yneg, &bc->zpos, &bc->zneg};
+  unsigned m = 0;
+  for (int f = 0; f < 6; f++) m |= (unsigned)(all[f]->type == OCU_BC_DIRICHELET) << f;
+  return m;
+}
+bool powers_of_two(const ocu_mg_level_params *p) {
+  int ex;
+  for (double f : {p->fx, p->fy, p->fz})
+    if (!(f > 0) || frexp(f, &ex) != 0.5 || ex < -60 || ex > 60) return false;
+  return true;
+}
+
+PairGeom pair_geom(const ocu_grid3d *u) {
+  PairGeom g;
+  g.nx = u->nx; g.ny = u->ny; g.nz = u->nz;
+  g.npz = (u->nz + 1) / 2;
+  g.n = u->nx * u->ny * g.npz;
+  g.my = mag(g.ny); g.mz = mag(g.nz); g.mpy = mag(g.ny + 2); g.mpz = mag(g.nz + 2);
+  g.mpair = mag(g.npz);
+  return g;
+}
+
+// Blocks when every level is exactly twice the next, faces are homogeneous
+// and cell pairs can be loaded as vectors; any other hierarchy that the
+// entry point accepts runs on k_mg_bottom.  Returns the LDS bytes, or 0.
+template <typename T, typename TC>
+size_t blocks_layout(const ocu_grid3d *u, const ocu_grid3d *b, int nlev, const ocu_bc_set *bc, BlkArgs<T, TC> &A) {
+  const int C = nlev - 1;
+  if (!plain_faces(bc, u, nlev) || !row_aligned(&b[0], 2)) return 0;
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    const size_t at = off;
+    off = (off + n + 15) & ~(size_t)15;
+    return (int)at;
+  };
+  for (int l = 0; l < C; l++) {
+    if (u[l].nx != 2 * u[l + 1].nx || u[l].ny != 2 * u[l + 1].ny || u[l].nz != 2 * u[l + 1].nz ||
+        !row_aligned(&u[l], 2))
+      return 0;
+    BlkLevel<T> &L = A.L[l];
+    L.u = dgrid<T>(&u[l]);
+    L.b = dgrid<T>(&b[l]);
+    L.bx = u[l + 1].nx; L.by = u[l + 1].ny; L.bz = u[l + 1].nz;
+    L.nb = L.bx * L.by * L.bz;
+    L.mby = mag(L.by); L.mbz = mag(L.bz);
+    L.my = mag(u[l].ny); L.mz = mag(u[l].nz); L.mpy = mag(u[l].ny + 2); L.mpz = mag(u[l].nz + 2);
+    L.toff = take(FACE_CLASSES * sizeof(Recip<T>));
+    L.uoff = take((size_t)L.nb * BLK * sizeof(T));
+    L.boff = take((size_t)L.nb * BLK * sizeof(T));
+  }
+  A.cu = dgrid<T>(&u[C]);
+  A.cb = dgrid<T>(&b[C]);
+  A.cg = pair_geom(&u[C]);
+  A.ctoff = take(FACE_CLASSES * sizeof(Recip<TC>));
+  A.cuoff = take(2 * (size_t)A.cg.n * sizeof(TC));
+  A.cboff = take(2 * (size_t)A.cg.n * sizeof(TC));
+  return off;
+}
+
 template <typename T, typename TC, int MODE>
 int launch_bottom(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p, const double *h, int nlev,
                   const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters, int zero_top, hipStream_t stream) {
+  BlkArgs<T, TC> K;
+  memset(&K, 0, sizeof(K));
+  const size_t blk_bytes = blocks_layout(u, b, nlev, bc, K);
+  if (blk_bytes && blk_bytes <= BOT_LDS_MAX) {
+    for (int l = 0; l + 1 < nlev; l++) {
+      K.L[l].dc = dev_c<T>(&p[l]);
+      K.L[l].rc = res_c<T>(p[l].h, p[l].fx, p[l].fy, p[l].fz);
+    }
+    K.hc = host_c<TC>(&p[nlev - 1]);
+    K.per[0] = bc->xpos.type == OCU_BC_PERIODIC;
+    K.per[1] = bc->ypos.type == OCU_BC_PERIODIC;
+    K.per[2] = bc->zpos.type == OCU_BC_PERIODIC;
+    K.flip = dirichlet_faces(bc);
+    K.nlev = nlev;
+    K.nu1 = nu1;
+    K.nu2 = nu2;
+    K.zero_top = zero_top;
+    K.coarse_iters = coarse_iters;
+    K.pow2 = powers_of_two(&p[nlev - 1]);
+    // a thread per block of the top level and per pair of the coarsest
+    const int items = std::max(K.L[0].nb, K.cg.n);
+    const int threads = std::min(BOT_THREADS, (items + 63) / 64 * 64);
+    // half the threads may hold twice the registers: an FP64 block takes 164
+    // (up to 16^3), and spills 74 of them beyond 512 blocks (45 us against
+    // k_mg_bottom's 105 at 20x20x16 all the same)
+    auto kern = threads <= BOT_THREADS / 2
+                    ? (K.flip ? k_mg_bottom_blocks<T, TC, true, BOT_THREADS / 2> : k_mg_bottom_blocks<T, TC, false, BOT_THREADS / 2>)
+                    : (K.flip ? k_mg_bottom_blocks<T, TC, true, BOT_THREADS> : k_mg_bottom_blocks<T, TC, false, BOT_THREADS>);
+    OCU_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)blk_bytes));
+    kern<<<1, threads, blk_bytes, stream>>>(K);
+    OCU_HIP_LAUNCHED("ocu_mg_bottom_vcycle");
+  }
   BotArgs<T, TC> A;
   memset(&A, 0, sizeof(A));
   const size_t bytes = bottom_layout<T, TC>(u, nlev, MODE, &A);
@@ -2239,6 +3031,30 @@ int launch_bottom(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_p
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   k_mg_bottom<T, TC, MODE><<<1, BOT_THREADS, bytes, stream>>>(A);
   OCU_HIP_LAUNCHED("ocu_mg_bottom_vcycle");
+}
+
+// ocu_mg_coarse_relax on pairs of cells (homogeneous faces)
+template <typename TS, typename TC>
+int launch_pairs(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
+                        const ocu_mg_level_params *p, const ocu_bc_set *bc, size_t bytes, hipStream_t stream) {
+  PairArgs<TS, TC> A;
+  A.u = dgrid<TS>(u);
+  A.b = dgrid<TS>(b);
+  A.g = pair_geom(u);
+  A.c = host_c<TC>(p);
+  A.per[0] = bc->xpos.type == OCU_BC_PERIODIC;
+  A.per[1] = bc->ypos.type == OCU_BC_PERIODIC;
+  A.per[2] = bc->zpos.type == OCU_BC_PERIODIC;
+  A.flip = dirichlet_faces(bc);
+  A.iterations = iterations;
+  A.order = order;
+  A.pow2 = powers_of_two(p);
+  const int threads = std::min(BOT_THREADS, (A.g.n + 63) / 64 * 64);
+  auto kern = A.flip ? k_coarse_pairs<TS, TC, true> : k_coarse_pairs<TS, TC, false>;
+  OCU_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)bytes));
+  kern<<<1, threads, bytes, stream>>>(A);
+  OCU_HIP_LAUNCHED("ocu_mg_coarse_relax");
 }
 
 }  // namespace
@@ -2598,6 +3414,14 @@ int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations
   size_t tsize = (mode == 1 || u->dtype == OCU_F64) ? 8 : 4;
   size_t shmem = 2 * box * tsize;
   FacesS F = faces_s(bc);
+  if (plain_faces(bc, u, 1)) {
+    const size_t bytes = FACE_CLASSES * sizeof(Recip<double>) + 4 * (size_t)g.nx * g.ny * ((g.nz + 1) / 2) * tsize;
+    if (bytes <= BOT_LDS_MAX) {
+      if (mode == 1) return launch_pairs<float, double>(u, b, iterations, order, p, bc, bytes, S(stream));
+      return u->dtype == OCU_F64 ? launch_pairs<double, double>(u, b, iterations, order, p, bc, bytes, S(stream))
+                                 : launch_pairs<float, float>(u, b, iterations, order, p, bc, bytes, S(stream));
+    }
+  }
   if (shmem > BOT_LDS_MAX) return coarse_relax_global(u, b, g, box, iterations, order, p, F, hx, hy, hz, mode, stream);
   // dynamic LDS beyond 64 KiB is requested explicitly
   const void *kc = mode == 1 ? reinterpret_cast<const void *>(&k_coarse<float, double, 1>)
