@@ -271,6 +271,26 @@ int ocu_mg_prolong_bc(const ocu_grid3d *u_coarse, const ocu_grid3d *u_fine, int 
  * periodic x/y pairs with a non-periodic z on whole rows; else 0 */
 int ocu_mg_prolong_bc_ok(const ocu_grid3d *u_coarse, const ocu_grid3d *u_fine,
                          const ocu_bc_set *bc);
+/* Two red-black iterations (OCU_RELAX_DEVICE arithmetic, a level-1 fill after
+ * each, periodic axes filled between colours too) out of place in one launch,
+ * for levels where launches and latency count:
+ *   u_coarse non-null: first u_in += the prolongation of u_coarse (with the
+ *     reference's corner choice), u_in itself staying as it is;
+ *   b_coarse non-null: after them the residual's restriction goes to
+ *     b_coarse's interior, and with norm_ws (sum r^2, max|r|) partials as
+ *     ocu_mg_residual_restrict leaves them (at most NORM_PARTS tiles of 8^3);
+ *   flags: OCU_FUSED_ZERO_INPUT (u_in is the zero grid and is not read).
+ * u_out gets the result with its level-1 ghost layer.  u_in's and u_coarse's
+ * ghost layers are their level-1 fills and are not read.  Needs even sides,
+ * homogeneous Neumann / Dirichlet faces or periodic pairs, and rows aligned
+ * to two cells (ocu_mg_smooth2_ok; else OCU_ERR_UNSUPPORTED).  Bit for bit
+ * the separate calls' results (the norms to rounding). */
+int ocu_mg_smooth2(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b,
+                   const ocu_grid3d *u_coarse, const ocu_grid3d *b_coarse,
+                   const ocu_mg_level_params *p, const ocu_bc_set *bc, int flags,
+                   double *norm_ws, void *stream);
+int ocu_mg_smooth2_ok(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b,
+                      const ocu_bc_set *bc);
 /* The bottom of a V-cycle in one workgroup: levels top..top+nlev-1 (the
  * last the coarsest) of Sol_MultigridPressure3DDevice, held in LDS.  Does
  * what the per-level calls do on them (sol_mgpressure3d.cpp:184-239):

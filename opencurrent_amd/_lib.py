@@ -100,6 +100,8 @@ HIP_SIGS = {
     "ocu_mac_adjoint_normal": (I, [GP, GP, GP, BP, P]),
     "ocu_divergence_adjoint": (I, [GP, GP, GP, GP, I, I, I, D, D, D, P]),
     "ocu_gradient_adjoint": (I, [GP, GP, GP, GP, D, D, D, D, P]),
+    "ocu_mg_smooth2": (I, [GP, GP, GP, GP, GP, MP, BP, I, DP, P]),
+    "ocu_mg_smooth2_ok": (I, [GP, GP, GP, BP]),
     "ocu_mg_bottom_vcycle": (I, [GP, GP, MP, DP, I, BP, I, I, I, I, I, P]),
     "ocu_mg_bottom_lds_bytes": (C.c_size_t, [GP, I, I]),
     "ocu_mg_bottom_lds_max": (C.c_size_t, []),

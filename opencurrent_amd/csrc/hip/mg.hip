@@ -2533,6 +2533,352 @@ __global__ __launch_bounds__(BOT_THREADS) void k_coarse_pairs(PairArgs<TS, TC> A
   pair_store<SIGN>(A.u, uc, A.g, A.per, A.flip);
 }
 
+// ------------------------------------------------------------------------
+// two relaxation iterations in one launch, by tiles
+// ------------------------------------------------------------------------
+//
+// The levels between the bottom and the large ones are a handful of launches
+// of 5 to 8 us each per V-cycle, and almost all of that is latency: a launch,
+// a first load, a march of a few planes with a barrier each.  Here one launch
+// does a whole leg of a level: the pending prolongation (PRO), two red-black
+// iterations out of place, and (DOWN) the residual, its restriction and its
+// norms - bit for bit the separate launches' results.
+//
+// A workgroup writes a tile of 4x4x4 blocks of 2x2x2 cells (a coarse cell
+// each) and holds the 8x8x8 blocks around it, a thread per block as in
+// k_mg_bottom_blocks.  Four colour passes and the residual reach five cells
+// beyond the tile; colour pass n needs right values only where the distance
+// |di|+|dj|+|dk| to the tile is at most 4-n (DOWN: 5-n), so the box loses one
+// layer per pass and nothing outside it is computed.  For DOWN the cells at
+// distance five straight out from the tile's faces are 96 more blocks, the
+// ring, loaded (and prolonged) by threads whose own block lies in a corner of
+// the box that nothing needs.  A periodic axis wraps the block coordinates; a
+// level smaller than the box is simply held more than once.
+constexpr int TILE_OUT = 4, TILE_BOX = 8, TILE_THREADS = TILE_BOX * TILE_BOX * TILE_BOX;
+constexpr int TILE_RING = 6 * TILE_OUT * TILE_OUT;
+
+template <typename T>
+struct TileArgs {
+  // cell (0,0,0) and byte strides (a grid's bytes fit 31 bits)
+  const T *uin, *b, *uc;
+  T *uout, *bc;
+  int uxs, uys, bxs, bys, cxs, cys, fxs, fys;  // uin and uout, b, uc, bc
+  typename DevCFor<T>::type c;
+  ResC<T> rc;
+  int n[3];                // blocks of the level (two or more per axis)
+  Mag ty, tz;              // tiles along y and z
+  int ntiles;
+  int per[3];
+  unsigned flip;
+  int zero;
+  double *parts;  // DOWN: norm partials (NORM_PARTS pairs) or null
+};
+
+// distance in cells from box coordinate x (0..7) of a block's nearest cell
+// to the tile (blocks 2..5)
+__device__ __forceinline__ int tile_dist(int x) { return x < 2 ? 3 - 2 * x : x > 5 ? 2 * x - 11 : 0; }
+
+// the value at a byte offset (not negative: the address is base + 32 bits)
+template <typename V, typename T>
+__device__ __forceinline__ V &at_bytes(T *p, int off) {
+  return *reinterpret_cast<V *>(reinterpret_cast<char *>(p) + (unsigned)off);
+}
+template <typename V, typename T>
+__device__ __forceinline__ const V &at_bytes(const T *p, int off) {
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + (unsigned)off);
+}
+
+template <typename T, bool SIGN, bool PRO, bool DOWN>
+__global__ __launch_bounds__(TILE_THREADS, 4) void k_smooth_tile(TileArgs<T> A) {
+  constexpr int SLOTS = TILE_THREADS + (DOWN ? TILE_RING : 0), W = sizeof(T);
+  __shared__ T U[SLOTS * BLK];
+  __shared__ Recip<T> tab[FACE_CLASSES];
+  // coarse cells staged for the prolongation: blocks 0..7 (DOWN: and the
+  // ring, -1..8) and one more around, from t0 - CPAD on
+  constexpr int CPAD = DOWN ? 2 : 1, CBOX = TILE_BOX + 2 * CPAD;
+  __shared__ T C[PRO ? CBOX * CBOX * CBOX : 1];
+  __shared__ double sh[DOWN ? 2 : 1][DOWN ? TILE_OUT * TILE_OUT * TILE_OUT : 1];
+
+  // each XCD takes a contiguous run of tiles
+  const int per_xcd = gridDim.x / FXCD;
+  const int tile = (blockIdx.x % FXCD) * per_xcd + blockIdx.x / FXCD;
+  if (tile >= A.ntiles) {  // uniform per block
+    if (DOWN && A.parts && threadIdx.x < 2) A.parts[2 * blockIdx.x + threadIdx.x] = 0.0;
+    return;
+  }
+  const int row = mdiv(tile, A.tz), tk = tile - row * (int)A.tz.n, ti = mdiv(row, A.ty), tj = row - ti * (int)A.ty.n;
+
+  // this thread's block of the box (the plane is the wave's)
+  const int t = threadIdx.x;
+  const int x[3] = {__builtin_amdgcn_readfirstlane(t >> 6), (t >> 3) & 7, t & 7};
+  const int t0[3] = {TILE_OUT * ti - 2, TILE_OUT * tj - 2, TILE_OUT * tk - 2};
+  const int dist = tile_dist(x[0]) + tile_dist(x[1]) + tile_dist(x[2]);
+  // block coordinates on the level, wrapped on periodic axes (at least seven
+  // blocks there: one step is enough); 0 where the level has no such block
+  auto place = [&](const int (&y)[3], int (&h)[3]) -> int {
+    int ok = 1;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int v = t0[a] + y[a], lo = v < 0, hi = v >= A.n[a];
+      h[a] = v + (A.per[a] ? (lo ? A.n[a] : 0) - (hi ? A.n[a] : 0) : 0);
+      ok &= A.per[a] | ((lo | hi) ^ 1);
+    }
+    return ok;
+  };
+  // the block's u or b as four pairs along k, from the bytes at off
+  auto pairs = [&](const T *d, int xs, int ys, const int (&h)[3], Two<T> (&p)[4]) {
+    const int off = 2 * (h[0] * xs + h[1] * ys + h[2] * W);
+#pragma unroll
+    for (int q = 0; q < 4; q++) p[q] = at_bytes<Two<T>>(d, off + (q >> 1) * xs + (q & 1) * ys);
+  };
+  int g[3];
+  const int exists = place(x, g);
+  const bool loads = exists & (dist <= (DOWN ? 5 : 4)), relaxes = exists & (dist <= 4);
+
+  // all loads in flight together: the coarse box, u and b of the block, the
+  // ring
+  // PRO: the coarse cells around the box (and the ring), ghosts as the
+  // level-1 fill has them: 16 threads per row along k
+  constexpr int CROWS = CBOX * CBOX, PT = PRO ? (CROWS + TILE_THREADS / 16 - 1) / (TILE_THREADS / 16) : 1;
+  T cv[PT];
+  int cm[PT];
+  const int ck = t & 15;
+  if (PRO) {
+    // one cell beyond a face is the ghost; further out is not read
+    auto coarse = [&](int a, int c, int &m) {
+      const int v = t0[a] - CPAD + c, lo = v < 0, hi = v >= A.n[a];
+      if (SIGN) m ^= (lo & (A.flip >> (2 * a + 1))) ^ (hi & (A.flip >> (2 * a)));
+      return A.per[a] ? v + (lo ? A.n[a] : 0) - (hi ? A.n[a] : 0) : min(max(v, 0), A.n[a] - 1);
+    };
+    int mk = 0;
+    const int offk = coarse(2, min(ck, CBOX - 1), mk) * W;
+#pragma unroll
+    for (int w = 0; w < PT; w++) {
+      const int r = min((t >> 4) + w * (TILE_THREADS / 16), CROWS - 1), ci = r / CBOX, cj = r - ci * CBOX;
+      cm[w] = mk;
+      const int off = coarse(0, ci, cm[w]) * A.cxs + coarse(1, cj, cm[w]) * A.cys + offk;
+      cv[w] = at_bytes<T>(A.uc, off);
+    }
+  }
+  Two<T> ru[4], rb[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) ru[q] = rb[q] = Two<T>{(T)0, (T)0};
+  if (loads) {
+    if (!A.zero) pairs(A.uin, A.uxs, A.uys, g, ru);
+    if (relaxes) pairs(A.b, A.bxs, A.bys, g, rb);
+  }
+  // DOWN: blocks of the box farther than five cells are not needed, and the
+  // 28 such threads of planes 0 and 7 each load the 96 ring blocks instead,
+  // one or two apiece (these waves sit out the last passes)
+  constexpr int IDLE = 56;
+  int rank = TILE_RING;
+  if (DOWN && (x[0] == 0 || x[0] == 7)) {
+    const unsigned long long idle = __ballot(dist > 5);
+    if (dist > 5)
+      rank = (x[0] ? 28 : 0) +
+             __builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0u));
+  }
+  auto ring_at = [&](int r, int (&y)[3]) {
+    const int f = r / 16, a = 2 + ((r >> 2) & 3), b = 2 + (r & 3), out = (f & 1) ? -1 : TILE_BOX;
+    y[0] = f < 2 ? out : a;
+    y[1] = f < 2 ? a : f < 4 ? out : b;
+    y[2] = f < 4 ? b : out;
+  };
+  auto put = [&](const Two<T> (&p)[4], int own) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      U[own + 2 * q] = p[q].a;
+      U[own + 2 * q + 1] = p[q].b;
+    }
+  };
+  Two<T> rz[2][4];
+  if (DOWN && rank < TILE_RING) {
+#pragma unroll
+    for (int w = 0; w < 2; w++) {
+      const int r = rank + w * IDLE;
+#pragma unroll
+      for (int q = 0; q < 4; q++) rz[w][q] = Two<T>{(T)0, (T)0};
+      int y[3], h[3];
+      ring_at(r, y);
+      if (!A.zero & (r < TILE_RING) & place(y, h)) pairs(A.uin, A.uxs, A.uys, h, rz[w]);
+    }
+  }
+  // (while the loads are on their way)
+  const int tq = t - TILE_THREADS / 2;
+  if (tq >= 0 && tq < FACE_CLASSES) tab[tq] = class_recip<T>(A.c, tq);
+  if (DOWN && rank < TILE_RING) {
+    put(rz[0], (TILE_THREADS + rank) * BLK);
+    if (rank + IDLE < TILE_RING) put(rz[1], (TILE_THREADS + rank + IDLE) * BLK);
+  }
+  if (PRO) {
+#pragma unroll
+    for (int w = 0; w < PT; w++) {
+      const int r = (t >> 4) + w * (TILE_THREADS / 16);
+      if (ck < CBOX && r < CROWS) C[r * CBOX + ck] = SIGN ? flip_sign(cv[w], (int)((unsigned)cm[w] << 31)) : cv[w];
+    }
+  }
+  if (PRO) __syncthreads();
+
+  // the prolongation of the coarse cells around block y to its u
+  auto prolong = [&](const int (&y)[3], T (&u)[8]) {
+    const T *c0 = &C[((y[0] + CPAD) * CBOX + y[1] + CPAD) * CBOX + y[2] + CPAD];
+    T v[3][3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) v[i][j][k] = c0[((i - 1) * CBOX + j - 1) * CBOX + k - 1];
+    blk_prolong(u, v);
+  };
+  Blk<T> s;
+  T b[8];
+  s.own = t * BLK;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    s.u[2 * q] = ru[q].a;
+    s.u[2 * q + 1] = ru[q].b;
+    b[2 * q] = rb[q].a;
+    b[2 * q + 1] = rb[q].b;
+  }
+  if (loads) {
+    if (PRO) prolong(x, s.u);
+#pragma unroll
+    for (int e = 0; e < 8; e++) U[s.own + e] = s.u[e];
+  }
+  if (PRO && DOWN && rank < TILE_RING) {
+    // the ring's blocks, one after the other (outside the level: unused)
+    for (int r = rank; r < TILE_RING; r += IDLE) {
+      int y[3];
+      T u[8];
+      ring_at(r, y);
+      const int own = (TILE_THREADS + r) * BLK;
+#pragma unroll
+      for (int e = 0; e < 8; e++) u[e] = U[own + e];
+      prolong(y, u);
+#pragma unroll
+      for (int e = 0; e < 8; e++) U[own + e] = u[e];
+    }
+  }
+  // face neighbours: the next block of the box, the ring, or the block's own
+  // cells (a level's face; also where the box ends and nothing needs them)
+  int cls[3][2];  // diagonal class of the low and high cells per axis
+  {
+    const int st[3] = {TILE_BOX * TILE_BOX, TILE_BOX, 1}, ch[3] = {4, 2, 1};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int p = a == 0 ? x[1] : x[0], q = a == 2 ? x[1] : x[2];  // in-plane box coordinates
+      const int mid = DOWN & ((unsigned)(p - 2) < 4u) & ((unsigned)(q - 2) < 4u);
+      const int ring = TILE_THREADS + 16 * 2 * a + 4 * (p - 2) + (q - 2);
+      const int lo = (A.per[a] ^ 1) & (g[a] == 0), hi = (A.per[a] ^ 1) & (g[a] == A.n[a] - 1);
+      const int out_hi = mid ? ring * BLK : s.own + ch[a], out_lo = mid ? (ring + 16) * BLK + ch[a] : s.own;
+      s.a[2 * a] = hi ? s.own + ch[a] : x[a] < TILE_BOX - 1 ? s.own + st[a] * BLK : out_hi;
+      s.a[2 * a + 1] = lo ? s.own : x[a] > 0 ? s.own - st[a] * BLK + ch[a] : out_lo;
+      if (SIGN) {
+        s.m[2 * a] = (int)((unsigned)(hi & (A.flip >> (2 * a))) << 31);
+        s.m[2 * a + 1] = (int)((unsigned)(lo & (A.flip >> (2 * a + 1))) << 31);
+      }
+      cls[a][0] = lo;
+      cls[a][1] = 2 * hi;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    s.hb[e] = b_term(A.c, b[e]);
+    s.q[e] = tab[(cls[0][e >> 2] * 3 + cls[1][(e >> 1) & 1]) * 3 + cls[2][e & 1]];
+  }
+  // passes 1..4
+  constexpr int reach = DOWN ? 4 : 3;
+  const int far = relaxes ? dist : 100;
+  if (far <= reach) blk_colour<SIGN, 0>(s, U, A.c);
+  __syncthreads();
+  if (far <= reach - 1) blk_colour<SIGN, 1>(s, U, A.c);
+  __syncthreads();
+  if (far <= reach - 2) blk_colour<SIGN, 0>(s, U, A.c);
+  __syncthreads();
+  if (far <= reach - 3) blk_colour<SIGN, 1>(s, U, A.c);
+  if (DOWN) __syncthreads();
+
+  double s2 = 0.0, mx = 0.0;
+  if (relaxes & (dist == 0) & (t0[0] + x[0] < A.n[0]) & (t0[1] + x[1] < A.n[1]) & (t0[2] + x[2] < A.n[2])) {
+    if (DOWN) {
+      T r[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        T zm, zp, ym, yp, xm, xp;
+        blk_nbrs<SIGN>(s, U, e, zm, zp, ym, yp, xm, xp);
+        r[e] = res_val(A.rc, b[e], zm, zp, ym, yp, xm, xp, s.u[e]);
+        if (A.parts) {
+          const double d = (double)r[e];
+          s2 += d * d;
+          mx = fmax(mx, fabs(d));
+        }
+      }
+      at_bytes<T>(A.bc, g[0] * A.fxs + g[1] * A.fys + g[2] * W) =
+          restrict_sum(r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]);
+    }
+    const int off = 2 * (g[0] * A.uxs + g[1] * A.uys + g[2] * W);
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      at_bytes<Two<T>>(A.uout, off + (q >> 1) * A.uxs + (q & 1) * A.uys) = Two<T>{s.u[2 * q], s.u[2 * q + 1]};
+    // the level-1 ghosts that derive from the block's cells (per axis the
+    // block lies at one end at most): `in` has the axes along which it does,
+    // end[a] the child bit of its cells there and to[a] the way to the ghosts
+    int end[3], to[3], ms[3], in = 0;
+    const int st[3] = {A.uxs, A.uys, W}, ch[3] = {4, 2, 1};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int lo = g[a] == 0, hi = g[a] == A.n[a] - 1;
+      in |= (lo | hi) << a;
+      end[a] = hi ? ch[a] : 0;
+      to[a] = (hi ? 2 : -1) * st[a];
+      if (A.per[a]) to[a] = (hi ? 1 - 2 * A.n[a] : 2 * A.n[a]) * st[a];
+      ms[a] = SIGN ? (int)((A.flip >> (hi ? 2 * a : 2 * a + 1)) << 31) : 0;
+    }
+    if (in) {
+#pragma unroll
+      for (int w = 1; w < 8; w++) {  // the axes a ghost lies beyond
+        if ((in & w) != w) continue;
+        int own = s.own, o = off, m = 0;
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+          if ((w >> a) & 1) own += end[a], o += to[a], m ^= ms[a];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {  // the block's cells at those ends
+          if ((((w & 1) << 2) | (w & 2) | ((w >> 2) & 1)) & e) continue;
+          const T v = U[own + e];
+          // (before cell (0,0,0): a signed offset)
+          *reinterpret_cast<T *>(reinterpret_cast<char *>(A.uout) +
+                                 (int64_t)(o + (e >> 2) * A.uxs + ((e >> 1) & 1) * A.uys + (e & 1) * W)) =
+              SIGN ? flip_sign(v, m) : v;
+        }
+      }
+    }
+  }
+  if (DOWN && A.parts) {  // uniform: the tile's 64 pairs through LDS to one wave
+    // (partials past the launch's blocks are zero)
+    for (int q = 2 * gridDim.x + tile * TILE_THREADS + t; q < 2 * NORM_PARTS; q += A.ntiles * TILE_THREADS)
+      A.parts[q] = 0.0;
+    if (dist == 0) {
+      const int q = ((x[0] - 2) * TILE_OUT + x[1] - 2) * TILE_OUT + x[2] - 2;
+      sh[0][q] = s2;
+      sh[1][q] = mx;
+    }
+    __syncthreads();
+    if (t < 64) {
+      s2 = sh[0][t];
+      mx = sh[1][t];
+      s2 = wave_sum(s2);
+      mx = wave_max(mx);
+      if (t == 0) {
+        A.parts[2 * blockIdx.x] = s2;
+        A.parts[2 * blockIdx.x + 1] = mx;
+      }
+    }
+  }
+}
+
 FacesS faces_s(const ocu_bc_set *bc) {
   FacesS F;
   const ocu_bc *all[6] = {&bc->xpos, &bc->xneg, &bc->ypos, &bc->yneg, &bc->zpos, &bc->zneg};
@@ -3057,9 +3403,102 @@ int launch_pairs(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int o
   OCU_HIP_LAUNCHED("ocu_mg_coarse_relax");
 }
 
+// Two iterations by tiles: every side even (2x2x2 blocks) and two blocks or
+// more, the faces of the block kernels, at least 14 cells along a periodic
+// axis (so that one step wraps the box) and rows that pairs of cells can be
+// loaded from.
+bool smooth_tile_ok(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b, const ocu_bc_set *bc) {
+  const int n[3] = {u_in->nx, u_in->ny, u_in->nz};
+  const int per[3] = {bc->xpos.type == OCU_BC_PERIODIC, bc->ypos.type == OCU_BC_PERIODIC,
+                      bc->zpos.type == OCU_BC_PERIODIC};
+  for (int a = 0; a < 3; a++)
+    if (n[a] % 2 || n[a] < 4 || (per[a] && n[a] < 14)) return false;
+  // (the tile's number is decoded by mdiv)
+  if ((int64_t)((n[0] + 7) / 8) * ((n[1] + 7) / 8) * ((n[2] + 7) / 8) >= 1 << 15) return false;
+  for (const ocu_grid3d *g : {u_in, b})  // byte offsets of cells fit an int
+    if (g->allocated >= (int64_t)INT_MAX / 8) return false;
+  return plain_faces(bc, u_in, 1) && row_aligned(u_in, 2) && row_aligned(u_out, 2) && row_aligned(b, 2);
+}
+
+template <typename T>
+int launch_smooth_tile(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b, const ocu_grid3d *uc,
+                       const ocu_grid3d *bc_out, const ocu_mg_level_params *p, const ocu_bc_set *bc, int zero,
+                       double *norm_ws, hipStream_t stream) {
+  TileArgs<T> A;
+  auto first = [](const ocu_grid3d *g) { return (T *)g->base + g->shift; };
+  auto xs = [](const ocu_grid3d *g) { return (int)((int64_t)g->pny * g->pnz * sizeof(T)); };
+  auto ys = [](const ocu_grid3d *g) { return (int)(g->pnz * sizeof(T)); };
+  const ocu_grid3d *c = uc ? uc : u_in, *f = bc_out ? bc_out : u_in;
+  A.uin = first(u_in); A.uout = first(u_out);
+  A.uxs = xs(u_in); A.uys = ys(u_in);
+  A.b = first(b); A.bxs = xs(b); A.bys = ys(b);
+  A.uc = first(c); A.cxs = xs(c); A.cys = ys(c);
+  A.bc = first(f); A.fxs = xs(f); A.fys = ys(f);
+  A.c = dev_c<T>(p);
+  A.rc = res_c<T>(p->h, p->fx, p->fy, p->fz);
+  A.n[0] = u_in->nx / 2; A.n[1] = u_in->ny / 2; A.n[2] = u_in->nz / 2;
+  const int tx = (A.n[0] + TILE_OUT - 1) / TILE_OUT;
+  A.ty = mag((A.n[1] + TILE_OUT - 1) / TILE_OUT);
+  A.tz = mag((A.n[2] + TILE_OUT - 1) / TILE_OUT);
+  A.ntiles = tx * (int)(A.ty.n * A.tz.n);
+  A.per[0] = bc->xpos.type == OCU_BC_PERIODIC;
+  A.per[1] = bc->ypos.type == OCU_BC_PERIODIC;
+  A.per[2] = bc->zpos.type == OCU_BC_PERIODIC;
+  A.flip = dirichlet_faces(bc);
+  A.zero = zero;
+  A.parts = norm_ws;
+  const int nblocks = ((A.ntiles + FXCD - 1) / FXCD) * FXCD;
+  void (*kern)(TileArgs<T>);
+#define OCU_TILE(PRO, DOWN) (A.flip ? k_smooth_tile<T, true, PRO, DOWN> : k_smooth_tile<T, false, PRO, DOWN>)
+  if (uc) kern = bc_out ? OCU_TILE(true, true) : OCU_TILE(true, false);
+  else kern = bc_out ? OCU_TILE(false, true) : OCU_TILE(false, false);
+#undef OCU_TILE
+  kern<<<nblocks, TILE_THREADS, 0, stream>>>(A);
+  OCU_HIP_LAUNCHED("ocu_mg_smooth2");
+}
+
 }  // namespace
 
 extern "C" {
+
+int ocu_mg_smooth2_ok(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b, const ocu_bc_set *bc) {
+  if (!u_in || !u_out || !b || !bc || check_pair(u_in, b, "ocu_mg_smooth2_ok") ||
+      check_grid(u_out, "ocu_mg_smooth2_ok"))
+    return 0;
+  return smooth_tile_ok(u_in, u_out, b, bc) ? 1 : 0;
+}
+
+int ocu_mg_smooth2(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_grid3d *b, const ocu_grid3d *u_coarse,
+                   const ocu_grid3d *b_coarse, const ocu_mg_level_params *p, const ocu_bc_set *bc, int flags,
+                   double *norm_ws, void *stream) {
+  const char *what = "ocu_mg_smooth2";
+  if (int e = check_pair(u_in, b, what)) return e;
+  if (int e = check_grid(u_out, "ocu_mg_smooth2(out)")) return e;
+  OCU_REQUIRE(p && bc, "%s: null argument", what);
+  OCU_REQUIRE(layout_match(u_in, u_out) && u_in->dtype == u_out->dtype && u_in->nx == u_out->nx &&
+                  u_in->ny == u_out->ny && u_in->nz == u_out->nz,
+              "%s: u_out must be congruent with u_in", what);
+  OCU_REQUIRE(u_out->gx >= 1 && u_out->gy >= 1 && u_out->gz >= 1, "%s: u_out needs one ghost layer", what);
+  OCU_REQUIRE((flags & ~OCU_FUSED_ZERO_INPUT) == 0, "%s: bad flags %d", what, flags);
+  const bool zero = flags & OCU_FUSED_ZERO_INPUT;
+  OCU_REQUIRE(u_in->base != u_out->base, "%s: u_out must not alias u_in", what);
+  OCU_REQUIRE(!norm_ws || b_coarse, "%s: the norms come with the restriction", what);
+  for (const ocu_grid3d *g : {u_coarse, b_coarse}) {
+    if (!g) continue;
+    if (int e = check_grid(g, what)) return e;
+    OCU_REQUIRE(g->dtype == u_in->dtype && u_in->nx == 2 * g->nx && u_in->ny == 2 * g->ny && u_in->nz == 2 * g->nz,
+                "%s: the coarse grids must be half of u", what);
+  }
+  if (!smooth_tile_ok(u_in, u_out, b, bc)) {
+    set_error("%s: needs even sides, homogeneous Neumann, Dirichlet or paired periodic faces and aligned rows", what);
+    return OCU_ERR_UNSUPPORTED;
+  }
+  const int64_t tiles = (int64_t)((u_in->nx + 7) / 8) * ((u_in->ny + 7) / 8) * ((u_in->nz + 7) / 8);
+  OCU_REQUIRE(!norm_ws || tiles <= NORM_PARTS, "%s: more tiles than norm partials", what);
+  return u_in->dtype == OCU_F64
+             ? launch_smooth_tile<double>(u_in, u_out, b, u_coarse, b_coarse, p, bc, zero, norm_ws, S(stream))
+             : launch_smooth_tile<float>(u_in, u_out, b, u_coarse, b_coarse, p, bc, zero, norm_ws, S(stream));
+}
 
 size_t ocu_mg_bottom_lds_max(void) { return BOT_LDS_MAX; }
 

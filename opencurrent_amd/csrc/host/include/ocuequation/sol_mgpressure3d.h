@@ -145,6 +145,14 @@ class Sol_MultigridPressure3DDevice : public Sol_MultigridPressure3DBase {
   // the fused sweep runs at level l (every face Neumann/Dirichlet, or the
   // periodic pairs it takes)
   bool _fused_lvl[kMaxLevels];
+  // _u_rlx[l]: two red-black iterations of level l (after its pending clear
+  // or prolongation) are pending: the residual and restriction that follow
+  // join them in one launch by tiles, and anything else that reads level l,
+  // or writes level l+1 before a pending prolongation, runs them first
+  bool _u_rlx[kMaxLevels];
+  // that launch is out of place, and u and its second buffer change places
+  // after it; _swapped[l]: they have done so an odd number of times
+  bool _swapped[kMaxLevels];
 
   Grid3DDevice<T> &get_u(int level) { return *_u_grid[level]; }
   Grid3DDevice<T> &get_r(int level) { return *_r_grid[level]; }
@@ -166,10 +174,17 @@ class Sol_MultigridPressure3DDevice : public Sol_MultigridPressure3DBase {
   void relax_colour_bc(int level, int color);
   bool relax_bc_ok(int level) const;
   void relax_coarsest(int level, int iterations, RelaxOrder order);
-  bool defer_ok(int level) const;
+  bool defer_ok(int level);
   void materialize(int level);
   void run_prolong(int coarse_level, int fine_level);
   // level l is about to change: a pending prolongation that reads it runs first
+  // the launch by tiles is the faster one at this level
+  bool tile_ok(int level);
+  void run_tile(int level, int coarse_level, bool norms);
+  void swap_buffers(int level);
+  bool prolong_sweep_ok(int level);
+  char level_state(int l) const;
+  void set_level_state(int l, char s);
   void flush_reader(int level) {
     if (level >= 1 && _u_pro[level - 1]) materialize(level - 1);
   }

@@ -354,7 +354,7 @@ Sol_MultigridPressure3DDevice<T>::Sol_MultigridPressure3DDevice() {
   _norm_tag = 0;
   _capturing = false;
   level0_sweeps[0] = level0_sweeps[1] = level0_sweeps[2] = 0;
-  for (int l = 0; l < kMaxLevels; l++) _u_zero[l] = _u_pro[l] = _fused_lvl[l] = false;
+  for (int l = 0; l < kMaxLevels; l++) _u_zero[l] = _u_pro[l] = _fused_lvl[l] = _u_rlx[l] = _swapped[l] = false;
 }
 
 template <typename T>
@@ -413,16 +413,69 @@ void Sol_MultigridPressure3DDevice<T>::level_params(int level, void *out) const 
 // A cleared level may stay unwritten when its next use is the fused
 // relaxation, which can start from the zero grid without reading it.
 template <typename T>
-bool Sol_MultigridPressure3DDevice<T>::defer_ok(int level) const {
-  if (!(use_fused_relax && _fused_lvl[level] && level < _num_levels - 1 && nu1 >= 2)) return false;
+bool Sol_MultigridPressure3DDevice<T>::defer_ok(int level) {
+  if (!(use_fused_relax && level < _num_levels - 1 && nu1 >= 2)) return false;
+  if (!_fused_lvl[level] && !(nu1 == 2 && tile_ok(level))) return false;
   // the zero grid's ghosts are all zero only for homogeneous faces
   BoundaryConditionSet lbc = get_bc_at_level(level);
   return lbc.xpos.value == 0 && lbc.xneg.value == 0 && lbc.ypos.value == 0 && lbc.yneg.value == 0 &&
          lbc.zpos.value == 0 && lbc.zneg.value == 0;
 }
 
+// Two iterations in one launch by tiles (ocu_mg_smooth2) cost three to eight
+// times the cell updates of two fused sweeps but one launch and one trip to
+// memory; measured with the restriction (prolongation): FP32 32^3 12.8 -> 7.0
+// us (13.6 -> 7.4), 64^3 14.7 -> 8.1 (15.6 -> 8.3), 96x80x112 20.0 -> 16.0
+// (22.6 -> 15.7), 128^3 26.9 -> 30.8 (30.4 -> 29.6); FP64 32^3 14.7 -> 7.9
+// (16.3 -> 8.0), 64^3 17.4 -> 9.4 (19.1 -> 10.4), 96x80x112 24.6 -> 24.8
+// (28.2 -> 26.1), 128^3 37.0 -> 51.8.  So up to 2^20 cells in FP32 and 3/4 of
+// that in FP64.  Where the fused sweep does not run (periodic z, 13 us a
+// colour at 128^3 in FP32) the tiles are the faster ones at any size they take.
+template <typename T>
+bool Sol_MultigridPressure3DDevice<T>::tile_ok(int level) {
+  if (!use_fused_relax || store_residuals || level >= _num_levels - 1) return false;
+  const long long cells = (long long)nx(level) * ny(level) * nz(level);
+  if (_fused_lvl[level] && cells > (sizeof(T) == 8 ? 3ll << 18 : 1ll << 20)) return false;
+  ocu_bc_set cbc = to_c_bc(get_bc_at_level(level));
+  ocu_grid3d u = get_u(level).desc(), a = _u_alt[level]->desc(), b = get_b(level).desc();
+  return ocu_mg_smooth2_ok(&u, &a, &b, &cbc) == 1;
+}
+
+template <typename T>
+void Sol_MultigridPressure3DDevice<T>::swap_buffers(int level) {
+  check_ok(get_u(level).swap_storage(*_u_alt[level]));
+  _swapped[level] = !_swapped[level];
+}
+
+// the pending iterations of a level (with its pending clear or
+// prolongation), and the residual and restriction to coarse_level if >= 0
+template <typename T>
+void Sol_MultigridPressure3DDevice<T>::run_tile(int level, int coarse_level, bool norms) {
+  const bool zero = _u_zero[level], pro = _u_pro[level];
+  _u_rlx[level] = _u_zero[level] = _u_pro[level] = false;
+  if (level == 0) {
+    level0_sweeps[pro ? 2 : zero ? 1 : 0]++;
+    level0_sweeps[0]++;
+  }
+  ocu_mg_level_params p;
+  level_params(level, &p);
+  ocu_bc_set cbc = to_c_bc(get_bc_at_level(level));
+  ocu_grid3d u = get_u(level).desc(), a = _u_alt[level]->desc(), b = get_b(level).desc(), uc, bc;
+  if (pro) uc = get_u(level + 1).desc();
+  if (coarse_level >= 0) bc = get_b(coarse_level).desc();
+  ok_status(ocu_mg_smooth2(&u, &a, &b, pro ? &uc : nullptr, coarse_level >= 0 ? &bc : nullptr, &p, &cbc,
+                           zero ? OCU_FUSED_ZERO_INPUT : 0, norms ? _norm_ws : nullptr,
+                           ThreadManager::get_compute_stream()),
+            "Sol_MultigridPressure3DDevice::relax");
+  swap_buffers(level);
+}
+
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::materialize(int level) {
+  if (_u_rlx[level]) {
+    run_tile(level, -1, false);
+    return;
+  }
   if (_u_pro[level]) {
     _u_pro[level] = false;
     run_prolong(level + 1, level);
@@ -436,6 +489,11 @@ void Sol_MultigridPressure3DDevice<T>::materialize(int level) {
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::settle() {
   for (int l = 0; l < _num_levels; l++) materialize(l);
+  // callers hold level 0's buffer (pressure())
+  if (_swapped[0]) {
+    check_ok(_u_alt[0]->copy_all_data(get_u(0)));
+    swap_buffers(0);
+  }
 }
 
 template <typename T>
@@ -454,6 +512,14 @@ void Sol_MultigridPressure3DDevice<T>::bottom_vcycle(int top) {
   ocu_grid3d u[kMaxLevels], b[kMaxLevels];
   ocu_mg_level_params p[kMaxLevels];
   double h[3 * kMaxLevels];
+  for (int l = top; l <= C; l++) {
+    if (_u_rlx[l]) materialize(l);
+    if (_u_pro[l]) {  // (a deferred zero stays deferred: the bottom takes it as a flag)
+      _u_pro[l] = false;
+      run_prolong(l + 1, l);
+    }
+    flush_reader(l);
+  }
   for (int l = 0; l < nlev; l++) {
     u[l] = get_u(top + l).desc();
     b[l] = get_b(top + l).desc();
@@ -461,13 +527,6 @@ void Sol_MultigridPressure3DDevice<T>::bottom_vcycle(int top) {
     h[3 * l] = hx(top + l);
     h[3 * l + 1] = hy(top + l);
     h[3 * l + 2] = hz(top + l);
-  }
-  for (int l = top; l <= C; l++) {
-    if (_u_pro[l]) {  // (a deferred zero stays deferred: the bottom takes it as a flag)
-      _u_pro[l] = false;
-      run_prolong(l + 1, l);
-    }
-    flush_reader(l);
   }
   ocu_bc_set cbc = to_c_bc(get_bc_at_level(top));
   int coarse_iters = max3(nx(C) * ny(C), ny(C) * nz(C), nx(C) * nz(C)) / 2;
@@ -480,7 +539,10 @@ void Sol_MultigridPressure3DDevice<T>::bottom_vcycle(int top) {
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::clear_zero(int level) {
   flush_reader(level);
-  _u_pro[level] = false;  // the grid becomes zero: the pending correction is moot
+  // the grid becomes zero: what is pending is moot, and so is which of the
+  // two buffers holds it
+  _u_pro[level] = _u_rlx[level] = false;
+  if (level > 0 && _swapped[level]) swap_buffers(level);
   if (defer_ok(level)) {
     _u_zero[level] = true;
     return;
@@ -492,7 +554,7 @@ void Sol_MultigridPressure3DDevice<T>::clear_zero(int level) {
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::apply_boundary_conditions(int level) {
   if (_u_zero[level]) return;  // the deferred zero grid carries its ghosts
-  if (_u_pro[level]) return;   // the pending prolongation writes them
+  if (_u_pro[level] || _u_rlx[level]) return;  // what is pending writes them
   flush_reader(level);
   if (!apply_3d_boundary_conditions_level1(get_u(level), get_bc_at_level(level), hx(level), hy(level), hz(level))) {
     printf("[ERROR] Sol_MultigridPressure3DDevice::apply_boundary_conditions - failed at level %d \n", level);
@@ -578,10 +640,16 @@ void Sol_MultigridPressure3DDevice<T>::relax(int level, int iterations, RelaxOrd
   };
 
   flush_reader(level);
+  if (_u_rlx[level]) materialize(level);
   if (iterations <= 0) {
     materialize(level);
     return;
   }
+  if (iterations == 2 && order == RO_RED_BLACK && tile_ok(level)) {
+    _u_rlx[level] = true;
+    return;
+  }
+  if (_u_pro[level] && !prolong_sweep_ok(level)) materialize(level);
   if (use_fused_relax && _fused_lvl[level]) {
     // pairs of out-of-place sweeps u -> alt -> u, so the result always ends
     // in u; each sweep also writes the level-1 ghosts of its output (the
@@ -657,11 +725,18 @@ void Sol_MultigridPressure3DDevice<T>::restrict_residuals(int fine_level, int co
 
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::restrict_residuals_launch(int fine_level, int coarse_level, bool norms) {
-  materialize(fine_level);
   void *s = ThreadManager::get_compute_stream();
+  if (coarse_level != fine_level && _u_rlx[coarse_level]) materialize(coarse_level);  // (they read its b)
+  // the pending iterations take the restriction (and norms, a partial pair
+  // per tile of 8^3 cells) along
+  const long long tiles = (long long)((nx(fine_level) + 7) / 8) * ((ny(fine_level) + 7) / 8) * ((nz(fine_level) + 7) / 8);
+  const bool joined = _u_rlx[fine_level] && coarse_level == fine_level + 1 && (!norms || tiles <= ocu_norm_parts());
+  if (joined) run_tile(fine_level, coarse_level, norms);
+  else materialize(fine_level);
   ocu_grid3d u = get_u(fine_level).desc(), b = get_b(fine_level).desc(), r = get_r(fine_level).desc();
   double h = get_h(fine_level);
-  if (coarse_level != fine_level) {
+  if (joined) {
+  } else if (coarse_level != fine_level) {
     ocu_grid3d bc = get_b(coarse_level).desc();
     ok_status(ocu_mg_residual_restrict(&u, &b, store_residuals ? &r : nullptr, &bc, h, _fx, _fy, _fz,
                                        norms ? _norm_ws : nullptr, s),
@@ -719,8 +794,21 @@ std::vector<long long> Sol_MultigridPressure3DDevice<T>::segment_key(void *strea
     k.push_back(v);
     k.push_back(a);
   }
-  for (int l = 0; l < _num_levels; l++) k.push_back(_u_zero[l] | _u_pro[l] << 1);
+  for (int l = 0; l < _num_levels; l++) k.push_back(level_state(l));
   return k;
+}
+
+// a level's pending work and which of its two buffers holds u
+template <typename T>
+char Sol_MultigridPressure3DDevice<T>::level_state(int l) const {
+  return (char)(_u_zero[l] | _u_pro[l] << 1 | _u_rlx[l] << 2 | _swapped[l] << 3);
+}
+template <typename T>
+void Sol_MultigridPressure3DDevice<T>::set_level_state(int l, char s) {
+  _u_zero[l] = s & 1;
+  _u_pro[l] = (s >> 1) & 1;
+  _u_rlx[l] = (s >> 2) & 1;
+  if (_swapped[l] != ((s >> 3) & 1)) swap_buffers(l);
 }
 
 template <typename T>
@@ -744,10 +832,7 @@ void Sol_MultigridPressure3DDevice<T>::run_segment(const std::function<void()> &
   for (Segment &g : _segments) {
     if (g.key != key) continue;
     if (!ok_status(ocu_graph_launch(g.exec, s), "Sol_MultigridPressure3DDevice::run_segment")) return;
-    for (int l = 0; l < _num_levels; l++) {
-      _u_zero[l] = g.out[l] & 1;
-      _u_pro[l] = (g.out[l] >> 1) & 1;
-    }
+    for (int l = 0; l < _num_levels; l++) set_level_state(l, g.out[l]);
     for (int q = 0; q < 3; q++) level0_sweeps[q] += g.sweeps[q];
     _norms_pending = true;
     _norm_tag = 0;
@@ -755,8 +840,8 @@ void Sol_MultigridPressure3DDevice<T>::run_segment(const std::function<void()> &
     return;
   }
   // the state to return to if the recording fails
-  std::vector<char> z(_num_levels), p(_num_levels);
-  for (int l = 0; l < _num_levels; l++) z[l] = _u_zero[l], p[l] = _u_pro[l];
+  std::vector<char> before(_num_levels);
+  for (int l = 0; l < _num_levels; l++) before[l] = level_state(l);
   long long sw[3] = {level0_sweeps[0], level0_sweeps[1], level0_sweeps[2]};
   const bool pending = _norms_pending, err = any_error();
   const unsigned long long tag = _norm_tag;
@@ -770,7 +855,7 @@ void Sol_MultigridPressure3DDevice<T>::run_segment(const std::function<void()> &
   }
   if (!ok) {
     if (exec) ocu_graph_destroy(exec);
-    for (int l = 0; l < _num_levels; l++) _u_zero[l] = z[l], _u_pro[l] = p[l];
+    for (int l = 0; l < _num_levels; l++) set_level_state(l, before[l]);
     for (int q = 0; q < 3; q++) level0_sweeps[q] = sw[q];
     _norms_pending = pending;
     _norm_tag = tag;
@@ -782,7 +867,7 @@ void Sol_MultigridPressure3DDevice<T>::run_segment(const std::function<void()> &
   Segment g;
   g.key = key;
   g.out.resize(_num_levels);
-  for (int l = 0; l < _num_levels; l++) g.out[l] = (char)(_u_zero[l] | _u_pro[l] << 1);
+  for (int l = 0; l < _num_levels; l++) g.out[l] = level_state(l);
   for (int q = 0; q < 3; q++) g.sweeps[q] = level0_sweeps[q] - sw[q];
   g.exec = exec;
   if (_segments.size() >= 4) {
@@ -799,15 +884,24 @@ void Sol_MultigridPressure3DDevice<T>::prolong(int coarse_level, int fine_level)
   materialize(coarse_level);
   materialize(fine_level);
   flush_reader(fine_level);
-  ocu_grid3d uc = get_u(coarse_level).desc(), uf = get_u(fine_level).desc();
-  if (use_fused_prolong && use_fused_relax && _fused_ok && coarse_level == fine_level + 1) {
-    ocu_bc_set cbc = to_c_bc(get_bc_at_level(fine_level));
-    if (ocu_mg_relax_fused_prolong_ok(&uf, &uc, &cbc)) {
-      _u_pro[fine_level] = true;  // the next fused relaxation of the fine level adds it
+  if (use_fused_prolong && use_fused_relax && coarse_level == fine_level + 1) {
+    // the next relaxation of the fine level adds it
+    const int next = fine_level > 0 ? nu2 : nu1;
+    if ((nu1 == 2 && next == 2 && tile_ok(fine_level)) || prolong_sweep_ok(fine_level)) {
+      _u_pro[fine_level] = true;
       return;
     }
   }
   run_prolong(coarse_level, fine_level);
+}
+
+// the fused sweep of this level can add the prolongation while it reads u
+template <typename T>
+bool Sol_MultigridPressure3DDevice<T>::prolong_sweep_ok(int level) {
+  if (!_fused_ok) return false;
+  ocu_bc_set cbc = to_c_bc(get_bc_at_level(level));
+  ocu_grid3d uc = get_u(level + 1).desc(), uf = get_u(level).desc();
+  return ocu_mg_relax_fused_prolong_ok(&uf, &uc, &cbc) == 1;
 }
 
 template <typename T>
@@ -841,7 +935,7 @@ bool Sol_MultigridPressure3DDevice<T>::initialize_storage(int nx_val, int ny_val
            nx_val, ny_val, nz_val);
     return false;
   }
-  for (int l = 0; l < kMaxLevels; l++) _u_zero[l] = _u_pro[l] = false;
+  for (int l = 0; l < kMaxLevels; l++) _u_zero[l] = _u_pro[l] = _u_rlx[l] = _swapped[l] = false;
   _update_bc_between_colors = bc.xpos.check_type(BC_PERIODIC) || bc.xneg.check_type(BC_PERIODIC) ||
                               bc.ypos.check_type(BC_PERIODIC) || bc.yneg.check_type(BC_PERIODIC) ||
                               bc.zpos.check_type(BC_PERIODIC) || bc.zneg.check_type(BC_PERIODIC);

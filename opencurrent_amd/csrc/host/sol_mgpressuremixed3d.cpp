@@ -246,6 +246,7 @@ bool Sol_MultigridPressureMixed3DDeviceD::do_fmg(double tolerance, int max_iter,
     }
     prev_res = res;
     _mg_f.relax(0, nu1, RO_RED_BLACK);
+    _mg_f.materialize(0);
     ocu_grid3d x = _x.desc(), e = _mg_f.pressure().desc();
     // singular problems: the correction also removes the interior mean of
     // x + e/s (from the residual pass's sum of x and one pass over e), so x
