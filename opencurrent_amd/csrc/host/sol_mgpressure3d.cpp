@@ -481,6 +481,7 @@ void Sol_MultigridPressure3DDevice<T>::materialize(int level) {
     run_prolong(level + 1, level);
   }
   if (!_u_zero[level]) return;
+  flush_reader(level);
   _u_zero[level] = false;
   check_ok(get_u(level).clear_zero());
   apply_boundary_conditions(level);
@@ -538,15 +539,18 @@ void Sol_MultigridPressure3DDevice<T>::bottom_vcycle(int top) {
 
 template <typename T>
 void Sol_MultigridPressure3DDevice<T>::clear_zero(int level) {
-  flush_reader(level);
-  // the grid becomes zero: what is pending is moot, and so is which of the
-  // two buffers holds it
+  // the grid becomes zero: what is pending is moot, and, unless the finer
+  // level still reads it, so is which of the two buffers holds it
   _u_pro[level] = _u_rlx[level] = false;
-  if (level > 0 && _swapped[level]) swap_buffers(level);
+  const bool read = level > 0 && _u_pro[level - 1];
+  if (level > 0 && _swapped[level] && !read) swap_buffers(level);
   if (defer_ok(level)) {
+    // (the buffer keeps what a pending prolongation reads until something
+    // writes it, which runs the reader first)
     _u_zero[level] = true;
     return;
   }
+  flush_reader(level);
   _u_zero[level] = false;
   check_ok(get_u(level).clear_zero());
 }
