@@ -9,6 +9,7 @@
 #include <climits>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "ghost_l1.h"
 #include "rows.h"
@@ -149,6 +150,84 @@ __device__ __forceinline__ T relax_pt_host(const HostC<T> &c, T uc, T zm, T zp, 
                                            T b, T x_mod, T y_mod, T z_mod) {
   return relax_pt_host_d(c, uc, zm, zp, ym, yp, xm, xp, b, diag_host(c, x_mod, y_mod, z_mod));
 }
+
+// ------------------------------------------------------------------------
+// division by a diagonal known in advance
+// ------------------------------------------------------------------------
+//
+// The relaxation divides by the diagonal, of which a level has 27 values
+// (none, low or high face per axis).  An IEEE division is about 11 VALU
+// instructions in FP32 and 14 in FP64 with a quarter-rate reciprocal in its
+// dependency chain; with the divisor's reciprocal at hand the same quotient,
+// bit for bit, takes 3 and 6:
+//   FP32: x times the double nearest 1/d, rounded once to float.  The double
+//     product is within 2^-52 (relative) of x/d, and a quotient of two floats
+//     keeps 2^-49 away from the middle between two floats (x = m*d with a
+//     25-bit odd m would need 25 bits in x), so the rounding is the
+//     quotient's; zeros, infinities and NaN come out as in a division, and a
+//     quotient below 2^-126 may end one denormal unit (1.4e-45) away.
+//   FP64: two fused corrections of x*r.  The first leaves a faithful
+//     quotient, whose remainder is exact, and by Markstein's theorem the
+//     second then rounds correctly, r being the correctly rounded 1/d;
+//     div_fixup gives the special operands their IEEE results.  (|x| below
+//     2^-960 would make the remainder inexact: one unit of a 1e-290 value.)
+template <typename T> struct Recip;
+template <> struct Recip<float> {
+  double r;
+};
+template <> struct Recip<double> {
+  double d, r;
+};
+__device__ __forceinline__ Recip<float> held(Recip<float> q) { return {held(q.r)}; }
+__device__ __forceinline__ Recip<double> held(Recip<double> q) { return {held(q.d), held(q.r)}; }
+__device__ __forceinline__ Recip<float> recip_of(float d) { return {1.0 / (double)d}; }
+__device__ __forceinline__ Recip<double> recip_of(double d) { return {d, 1.0 / d}; }
+__device__ __forceinline__ float div_by(float x, const Recip<float> &q) { return (float)((double)x * q.r); }
+__device__ __forceinline__ double div_by(double x, const Recip<double> &q) {
+  double y = x * q.r;
+  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
+  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
+  return __builtin_amdgcn_div_fixup(y, q.d, x);
+}
+
+// relax_pt with b's term and the diagonal's reciprocal in hand
+__device__ __forceinline__ double b_term(const DevC64 &c, double b) { return c.neg_hsq * b; }
+__device__ __forceinline__ float b_term(const DevC32 &c, float b) { return -c.hsq * b; }
+template <typename Q>
+__device__ __forceinline__ double relax_pt_q(const DevC64 &c, double uc, double zm, double zp, double ym, double yp,
+                                             double xm, double xp, double hb, const Q &q) {
+  double r = -c.ld * uc;
+  r += c.fz * (zm + zp);
+  r += c.fy * (ym + yp);
+  r += c.fx * (xm + xp);
+  r += hb;
+  return uc + div_by(c.omega * r, q);
+}
+template <typename Q>
+__device__ __forceinline__ float relax_pt_q(const DevC32 &c, float uc, float zm, float zp, float ym, float yp,
+                                            float xm, float xp, float hb, const Q &q) {
+  float r = (hb - c.ld * uc);
+  r += c.fz * (zm + zp);
+  r += c.fy * (ym + yp);
+  r += c.fx * (xm + xp);
+  return uc + div_by(c.omega * r, q);
+}
+
+// a divisor without its reciprocal: the plain division
+template <typename T> struct Diag {
+  T d;
+};
+template <typename T>
+__device__ __forceinline__ Diag<T> held(Diag<T> q) { return {held(q.d)}; }
+template <typename T>
+__device__ __forceinline__ T div_by(T x, const Diag<T> &q) { return x / q.d; }
+template <typename Q> struct Divisor;
+template <typename T> struct Divisor<Recip<T>> {
+  static __device__ __forceinline__ Recip<T> of(T d) { return recip_of(d); }
+};
+template <typename T> struct Divisor<Diag<T>> {
+  static __device__ __forceinline__ Diag<T> of(T d) { return {d}; }
+};
 
 // ------------------------------------------------------------------------
 // one colour, in place
@@ -351,10 +430,24 @@ __device__ __forceinline__ void write_ghost_row(const DGrid<T> &o, const GhostL1
 // merged into one with a computed element index, which sends the caller's
 // row to scratch memory.
 //
-// drow: the row's diagonal without the z ends (diag_row of the row's i and
-// j); the z ends go on top per cell, k = 0 only for e = 0 (k0 = V * lane).
-template <int P, typename T, int V, typename C>
-__device__ __forceinline__ Vec<T, V> relax_row_elems(const C &c, T drow, int kpar, int k0, int kupd, int nz,
+// q: the reciprocals of the diagonals of the lane's first cell, its last one
+// (the z ends are among them: k = 0 only for e = 0, k = nz-1 only for
+// e = V-1, since V divides nz) and those between.
+template <typename Q>
+struct RowQ {
+  Q first, mid, last;
+};
+// drow: the row's diagonal without the z ends (diag_row of the row's i and j)
+template <typename Q, int V, typename T, typename C>
+__device__ __forceinline__ RowQ<Q> row_q(const C &c, T drow, int k0, int nz) {
+  T d0 = drow, dl = drow;
+  if (V == 1 && k0 == nz - 1) d0 += c.m[4];
+  if (k0 == 0) d0 += c.m[5];
+  if (k0 + V == nz) dl += c.m[4];
+  return {Divisor<Q>::of(d0), held(Divisor<Q>::of(drow)), Divisor<Q>::of(dl)};
+}
+template <int P, typename T, int V, typename C, typename Q>
+__device__ __forceinline__ Vec<T, V> relax_row_elems(const C &c, const RowQ<Q> &q, int kpar, int k0, int kupd,
                                                      const Vec<T, V> &cen, T lo, T hi, const Vec<T, V> &ym,
                                                      const Vec<T, V> &yp, const Vec<T, V> &xm, const Vec<T, V> &xp,
                                                      const Vec<T, V> &b, Vec<T, V> out) {
@@ -363,25 +456,22 @@ __device__ __forceinline__ Vec<T, V> relax_row_elems(const C &c, T drow, int kpa
 #pragma unroll
   for (int m = 0; m < NE; m++) {
     const int e = P + S * m, k = k0 + e;
-    T d = drow;
-    if (k == nz - 1) d += c.m[4];
-    if (e == 0 && k == 0) d += c.m[5];
-    const T nv = relax_pt(c, cen.v[e], e > 0 ? cen.v[e - 1] : lo, e < V - 1 ? cen.v[e + 1] : hi, ym.v[e], yp.v[e],
-                          xm.v[e], xp.v[e], b.v[e], d);
+    const T nv = relax_pt_q(c, cen.v[e], e > 0 ? cen.v[e - 1] : lo, e < V - 1 ? cen.v[e + 1] : hi, ym.v[e], yp.v[e],
+                            xm.v[e], xp.v[e], b_term(c, b.v[e]), e == 0 ? q.first : e == V - 1 ? q.last : q.mid);
     const bool keep = V == 1 ? ((k & 1) == kpar && k < kupd) : k < kupd;
     out.v[e] = keep ? nv : out.v[e];
   }
   return out;
 }
-template <typename T, int V, typename C>
-__device__ __forceinline__ Vec<T, V> relax_row(const C &c, T drow, int kpar, int k0, int kupd, int nz,
+template <typename T, int V, typename C, typename Q>
+__device__ __forceinline__ Vec<T, V> relax_row(const C &c, const RowQ<Q> &q, int kpar, int k0, int kupd,
                                                const Vec<T, V> &cen, T lo, T hi, const Vec<T, V> &ym,
                                                const Vec<T, V> &yp, const Vec<T, V> &xm, const Vec<T, V> &xp,
                                                const Vec<T, V> &b, const Vec<T, V> &out) {
   static_assert(V == 1 || V % 2 == 0, "rows hold 1 or an even number of cells per lane");
   if (V == 1 || kpar == 0)
-    return relax_row_elems<0, T, V>(c, drow, kpar, k0, kupd, nz, cen, lo, hi, ym, yp, xm, xp, b, out);
-  return relax_row_elems<1, T, V>(c, drow, kpar, k0, kupd, nz, cen, lo, hi, ym, yp, xm, xp, b, out);
+    return relax_row_elems<0, T, V>(c, q, kpar, k0, kupd, cen, lo, hi, ym, yp, xm, xp, b, out);
+  return relax_row_elems<1, T, V>(c, q, kpar, k0, kupd, cen, lo, hi, ym, yp, xm, xp, b, out);
 }
 
 // Rows of a block: NW waves of R rows each; the outer two rows on each side
@@ -406,6 +496,15 @@ __device__ __forceinline__ Vec<T, V> relax_row(const C &c, T drow, int kpar, int
 #endif
 template <typename T, bool PRO>
 constexpr int fused_rows_min_waves() { return sizeof(T) == 4 ? (PRO ? OCU_ROWS_PRO_WAVES : OCU_ROWS_F32_WAVES) : 1; }
+
+// Divisions by reciprocals where their registers are free; the FP32 sweep with
+// the prolongation and the FP64 one with two cells per lane would lose the
+// second block of a CU to them, or spill (68 against 56.5 us at 256^3, 17.7
+// against 16.0 us at 128^3), and divide.  Elsewhere, plain (zero start): FP32
+// 256^3 40.2 -> 37.8 us (31.2 -> 27.5), FP64 100.4 -> 94.9 us (76.8 -> 70.7).
+template <typename T, int V, bool ZERO, bool PRO> struct RowsDivisor {
+  typedef typename std::conditional<sizeof(T) == 4 ? PRO : V == 2 && !ZERO, Diag<T>, Recip<T>>::type type;
+};
 
 // block barriers per plane of the whole-row sweep (1 or 2; the macro exists
 // for tuning builds)
@@ -479,7 +578,16 @@ __global__ __launch_bounds__(64 * NW, (fused_rows_min_waves<T, PRO>())) void k_r
     dhi[r] = held(diag_row<T>(c, nx - 1, jw[r], nx, ny));
     dmid[r] = held(diag_row<T>(c, -1, jw[r], nx, ny));
   }
-  auto drow = [&](int r, int i) { return i == 0 ? dlo[r] : i == nx - 1 ? dhi[r] : dmid[r]; };
+  // the reciprocals of the planes between, kept, and of a face plane, taken
+  // there (uniform)
+  typedef typename RowsDivisor<T, V, ZERO, PRO>::type Q;
+  RowQ<Q> qmid[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) qmid[r] = row_q<Q, V>(c, dmid[r], k0, nz);
+  auto rowq = [&](int r, int i) {
+    if (i == 0 || i == nx - 1) return row_q<Q, V>(c, i == 0 ? dlo[r] : dhi[r], k0, nz);
+    return qmid[r];
+  };
   auto plane_u = [&](int p) { return px ? wrap1(p, nx) : min(max(p, -1), nx); };
   auto plane_b = [&](int p) { return px ? wrap1(p, nx) : min(max(p, 0), nx - 1); };
   auto ring1 = [&](int r) { return t0 + r >= 1 && t0 + r <= NR - 2; };
@@ -709,8 +817,8 @@ __global__ __launch_bounds__(64 * NW, (fused_rows_min_waves<T, PRO>())) void k_r
         const int j = jw[r], pw = px ? wrap1(p, nx) : p;
         const VT ym = r > 0 ? cc[r > 0 ? r - 1 : 0] : sU0[u0slot(p)][t0 - 1][lane];
         const VT yp = r < R - 1 ? cc[r < R - 1 ? r + 1 : 0] : sU0[u0slot(p)][t0 + R][lane];
-        u1[r] = relax_row<T, V>(c, drow(r, pw), (first_color ^ pw ^ j) & 1, k0, kupd, nz, cc[r], lo, hi, ym, yp,
-                                u1m1[r], n[r], bcur[r], u1[r]);
+        u1[r] = relax_row<T, V>(c, rowq(r, pw), (first_color ^ pw ^ j) & 1, k0, kupd, cc[r], lo, hi, ym, yp, u1m1[r],
+                                n[r], bcur[r], u1[r]);
       }
       sU1[p & 1][t0 + r][lane] = u1[r];
     }
@@ -728,8 +836,8 @@ __global__ __launch_bounds__(64 * NW, (fused_rows_min_waves<T, PRO>())) void k_r
         const int j = jb + r;
         const VT ym = r > 0 ? u1m1[r > 0 ? r - 1 : 0] : sU1[q & 1][t0 - 1][lane];
         const VT yp = r < R - 1 ? u1m1[r < R - 1 ? r + 1 : 0] : sU1[q & 1][t0 + R][lane];
-        const VT v = relax_row<T, V>(c, drow(r, q), (first_color ^ q ^ j ^ 1) & 1, k0, kupd, nz, u1m1[r], lo, hi, ym,
-                                     yp, u1m2[r], u1[r], bprev[r], u1m1[r]);
+        const VT v = relax_row<T, V>(c, rowq(r, q), (first_color ^ q ^ j ^ 1) & 1, k0, kupd, u1m1[r], lo, hi, ym, yp,
+                                     u1m2[r], u1[r], bprev[r], u1m1[r]);
         if (active) {
           *reinterpret_cast<VT *>(uout.p + (int64_t)q * uout.xs + (int64_t)j * uout.ys + k0) = v;
           if (wghost) {  // ghosts of this row: z ends, x and y face rows
@@ -1849,43 +1957,6 @@ __global__ __launch_bounds__(BOT_THREADS) void k_mg_bottom(BotArgs<T, TC> args) 
 }
 
 // ------------------------------------------------------------------------
-// division by a diagonal known in advance
-// ------------------------------------------------------------------------
-//
-// The relaxation divides by the diagonal, of which a level has 27 values
-// (none, low or high face per axis).  An IEEE division is about 11 VALU
-// instructions in FP32 and 14 in FP64 with a quarter-rate reciprocal in its
-// dependency chain; with the divisor's reciprocal at hand the same quotient,
-// bit for bit, takes 3 and 6:
-//   FP32: x times the double nearest 1/d, rounded once to float.  The double
-//     product is within 2^-52 (relative) of x/d, and a quotient of two floats
-//     keeps 2^-49 away from the middle between two floats (x = m*d with a
-//     25-bit odd m would need 25 bits in x), so the rounding is the
-//     quotient's; zeros, infinities and NaN come out as in a division, and a
-//     quotient below 2^-126 may end one denormal unit (1.4e-45) away.
-//   FP64: two fused corrections of x*r.  The first leaves a faithful
-//     quotient, whose remainder is exact, and by Markstein's theorem the
-//     second then rounds correctly, r being the correctly rounded 1/d;
-//     div_fixup gives the special operands their IEEE results.  (|x| below
-//     2^-960 would make the remainder inexact: one unit of a 1e-290 value.)
-template <typename T> struct Recip;
-template <> struct Recip<float> {
-  double r;
-};
-template <> struct Recip<double> {
-  double d, r;
-};
-__device__ __forceinline__ Recip<float> recip_of(float d) { return {1.0 / (double)d}; }
-__device__ __forceinline__ Recip<double> recip_of(double d) { return {d, 1.0 / d}; }
-__device__ __forceinline__ float div_by(float x, const Recip<float> &q) { return (float)((double)x * q.r); }
-__device__ __forceinline__ double div_by(double x, const Recip<double> &q) {
-  double y = x * q.r;
-  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
-  y = __builtin_fma(__builtin_fma(-y, q.d, x), q.r, y);
-  return __builtin_amdgcn_div_fixup(y, q.d, x);
-}
-
-// ------------------------------------------------------------------------
 // the bottom of a V-cycle, a thread per coarse cell
 // ------------------------------------------------------------------------
 //
@@ -1982,27 +2053,6 @@ __device__ __forceinline__ Recip<T> class_recip(const C &c, int q) {
   if (y) d += c.m[y == 2 ? 2 : 3];
   if (z) d += c.m[z == 2 ? 4 : 5];
   return recip_of(d);
-}
-
-// relax_pt with b's term and the diagonal's reciprocal in hand
-__device__ __forceinline__ double b_term(const DevC64 &c, double b) { return c.neg_hsq * b; }
-__device__ __forceinline__ float b_term(const DevC32 &c, float b) { return -c.hsq * b; }
-__device__ __forceinline__ double relax_pt_q(const DevC64 &c, double uc, double zm, double zp, double ym, double yp,
-                                             double xm, double xp, double hb, const Recip<double> &q) {
-  double r = -c.ld * uc;
-  r += c.fz * (zm + zp);
-  r += c.fy * (ym + yp);
-  r += c.fx * (xm + xp);
-  r += hb;
-  return uc + div_by(c.omega * r, q);
-}
-__device__ __forceinline__ float relax_pt_q(const DevC32 &c, float uc, float zm, float zp, float ym, float yp,
-                                            float xm, float xp, float hb, const Recip<float> &q) {
-  float r = (hb - c.ld * uc);
-  r += c.fz * (zm + zp);
-  r += c.fy * (ym + yp);
-  r += c.fx * (xm + xp);
-  return uc + div_by(c.omega * r, q);
 }
 
 // a thread's block of a level: its cells (e = 4*dx + 2*dy + dz), b's terms,
