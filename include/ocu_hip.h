@@ -127,6 +127,11 @@ int ocu_bc_fill_level1(const ocu_grid3d *g, const ocu_bc_set *bc, double hx, dou
  * (grid3dboundary.cu:28-119, 719-753) */
 int ocu_bc_fill_nocorners(const ocu_grid3d *g, const ocu_bc_set *bc, double hx, double hy,
                           double hz, void *stream);
+/* r = a1*g1 + a2*g2 (ocu_grid_lincomb), then ocu_bc_fill_nocorners(r), in one
+ * launch unless ocu_grid_lincomb's rule covers the whole allocation */
+int ocu_grid_lincomb_fill(const ocu_grid3d *r, double a1, const ocu_grid3d *g1, double a2,
+                          const ocu_grid3d *g2, const ocu_bc_set *bc, double hx, double hy,
+                          double hz, void *stream);
 /* apply_3d_mac_boundary_conditions_level1 (grid3dboundary.cu:825-900) */
 int ocu_bc_fill_mac_level1(const ocu_grid3d *u, const ocu_grid3d *v, const ocu_grid3d *w,
                            const ocu_bc_set *bc, void *stream);
@@ -415,6 +420,30 @@ int ocu_passive_advect_adjoint(const ocu_grid3d *u, const ocu_grid3d *v, const o
                                const ocu_grid3d *adj_u, const ocu_grid3d *adj_v, const ocu_grid3d *adj_w,
                                double scale, int nx, int ny, int nz, double hx, double hy, double hz,
                                int scheme, void *stream);
+/* One step of the scalar transport in one launch:
+ *   phi_out = fill(phi + dt * A(u, phi))
+ * with A the passive advection (OCU_IT_FIRST_ORDER_UPWIND or
+ * OCU_IT_SECOND_ORDER_CENTERED) and fill the no-corner ghost fill of bc: the
+ * interior and the face ghosts of phi_out are what ocu_passive_advect,
+ * ocu_grid_lincomb and ocu_bc_fill_nocorners give, bit for bit; its edges,
+ * corners and padding are not written.  dphi is a scratch grid of the same
+ * layout: phi_out may be phi, and rows beyond 256 cells or not divisible over
+ * the lanes are taken, by those three calls. */
+int ocu_passive_advect_step(const ocu_grid3d *u, const ocu_grid3d *v, const ocu_grid3d *w,
+                            const ocu_grid3d *phi, const ocu_grid3d *phi_out,
+                            const ocu_grid3d *dphi, double dt, double hx, double hy, double hz,
+                            int scheme, const ocu_bc_set *bc, void *stream);
+/* Its adjoint with scale = dt: lam_out's interior is lam transported back with
+ * the adjoints of the face ghosts folded in (ocu_passive_advect_adjoint, then
+ * ocu_bc_adjoint_nocorners on lam_out), adj_u/v/w accumulate.  lam's ghost
+ * layer must be zero; lam_out's face ghosts are left as they are (by those two
+ * calls: zero). */
+int ocu_passive_advect_adjoint_step(const ocu_grid3d *u, const ocu_grid3d *v, const ocu_grid3d *w,
+                                    const ocu_grid3d *phi, const ocu_grid3d *lam,
+                                    const ocu_grid3d *lam_out, const ocu_grid3d *adj_u,
+                                    const ocu_grid3d *adj_v, const ocu_grid3d *adj_w, double scale,
+                                    double hx, double hy, double hz, int scheme,
+                                    const ocu_bc_set *bc, void *stream);
 /* Adjoint of ocu_bc_fill_nocorners: folds every face ghost's adjoint into
  * the interior cell it derives from (periodic/Neumann +1, Dirichlet -1,
  * BC_NONE dropped) and zeroes the face ghosts. */

@@ -71,6 +71,7 @@ HIP_SIGS = {
     "ocu_grid_maxabs3_tagged": (I, [GP, GP, GP, P, DP, C.c_ulonglong, P]),
     "ocu_grid_reduce_noalloc": (I, [GP, I, DP, P]),
     "ocu_bc_fill_level1": (I, [GP, BP, D, D, D, P]),
+    "ocu_grid_lincomb_fill": (I, [GP, D, GP, D, GP, BP, D, D, D, P]),
     "ocu_bc_fill_nocorners": (I, [GP, BP, D, D, D, P]),
     "ocu_bc_fill_mac_level1": (I, [GP, GP, GP, BP, P]),
     "ocu_bc_fill_level2_nocorners": (I, [GP, BP, D, D, D, P]),
@@ -96,6 +97,8 @@ HIP_SIGS = {
     "ocu_grid_clear_ghosts": (I, [GP, P]),
     "ocu_grid_stats3": (I, [GP, DP, P]),
     "ocu_passive_advect_adjoint": (I, [GP, GP, GP, GP, GP, GP, GP, GP, GP, D, I, I, I, D, D, D, I, P]),
+    "ocu_passive_advect_step": (I, [GP, GP, GP, GP, GP, GP, D, D, D, D, I, BP, P]),
+    "ocu_passive_advect_adjoint_step": (I, [GP, GP, GP, GP, GP, GP, GP, GP, GP, D, D, D, D, I, BP, P]),
     "ocu_bc_adjoint_nocorners": (I, [GP, BP, P]),
     "ocu_mac_adjoint_normal": (I, [GP, GP, GP, BP, P]),
     "ocu_divergence_adjoint": (I, [GP, GP, GP, GP, I, I, I, D, D, D, P]),

@@ -9,7 +9,7 @@ Eqn_ScalarAdvection3D::advance_one_step chains it, eqn_scalaradvection3d.cpp):
 
 with A the passive advection (Sol_PassiveAdvection3DDevice) and fill the
 device no-corner ghost fill.  The reference has no adjoint; this one is built
-from hand-written kernels of libocu_hip.so: ocu_passive_advect_adjoint,
+from hand-written kernels of libocu_hip.so: ocu_passive_advect_adjoint_step,
 ocu_bc_adjoint_nocorners, ocu_mac_adjoint_normal, ocu_gradient_adjoint,
 ocu_divergence_adjoint.  The projection P = M (I - G B S D) M (MAC fill M,
 divergence D, pressure solve S, pressure ghost fill B, gradient G) has the
@@ -111,7 +111,7 @@ class AdvectProjectProblem:
         self.lam, self.lam2 = D.DeviceGrid.congruent(like), D.DeviceGrid.congruent(like)
         nseg = (self.steps + self.ce - 1) // self.ce
         self.ck = [D.DeviceGrid.congruent(like) for _ in range(nseg)]
-        self.seg = [D.DeviceGrid.congruent(like) for _ in range(min(self.ce, self.steps))]
+        self.seg = [D.DeviceGrid.congruent(like) for _ in range(min(self.ce, self.steps) - 1)]
         self.masks = [parameter_mask(g, q) for q, g in enumerate((self.u, self.v, self.w))]
         self.loss = None
         # number of forward passes run; a gradient belongs to the forward
@@ -146,10 +146,7 @@ class AdvectProjectProblem:
         D.mac_adjoint_normal(self.au, self.av, self.aw, self.flow_bc)
 
     def _step(self, src, dst):
-        nx, ny, nz = self.n
-        D.passive_advect(self.u, self.v, self.w, src, self.dphi, nx, ny, nz, *self.h, self.scheme)
-        D.grid_lincomb(dst, 1.0, src, self.dt, self.dphi)
-        D.bc_fill_nocorners(dst, self.phi_bc, *self.h)
+        D.passive_advect_step(self.u, self.v, self.w, src, dst, self.dphi, self.dt, *self.h, self.scheme, self.phi_bc)
 
     def set_scalars(self, phi0, target):
         """initial scalar and target (tensors or arrays over the interior)"""
@@ -167,11 +164,15 @@ class AdvectProjectProblem:
             g.tensor.zero_()
             g.tensor[m] = x.detach().to(g.tensor.dtype)[m]
         self._project(self.proj)
-        D.grid_copy(self.phi, self.phi0)
-        for n in range(self.steps):
-            if n % self.ce == 0:
-                D.grid_copy(self.ck[n // self.ce], self.phi)
-            self._step(self.phi, self.phi)
+        # a state is written where it is kept: the checkpoints, and the last
+        # one in phi; those between alternate between phi and a backward buffer
+        last = self.ck[0] if self.steps else self.phi
+        D.grid_copy(last, self.phi0)
+        for n in range(1, self.steps + 1):
+            even = (self.steps - n) % 2 == 0
+            dst = self.ck[n // self.ce] if n % self.ce == 0 and n < self.steps else self.phi if even else self.lam2
+            self._step(last, dst)
+            last = dst
         self.seed.tensor.zero_()
         D.grid_lincomb(self.seed, 1.0, self.phi, -1.0, self.target)
         D.grid_clear_ghosts(self.seed)
@@ -192,15 +193,15 @@ class AdvectProjectProblem:
         D.grid_copy(lam, self.seed)
         for s in reversed(range(len(self.ck))):
             n0, n1 = s * self.ce, min(s * self.ce + self.ce, self.steps)
-            D.grid_copy(self.seg[0], self.ck[s])
+            seg = [self.ck[s]] + self.seg[:n1 - n0 - 1]
             for m in range(1, n1 - n0):
-                self._step(self.seg[m - 1], self.seg[m])
+                self._step(seg[m - 1], seg[m])
             for n in reversed(range(n0, n1)):
-                D.bc_adjoint_nocorners(lam, self.phi_bc)
-                D.passive_advect_adjoint(self.u, self.v, self.w, self.seg[n - n0], lam, lam2, self.au, self.av,
-                                         self.aw, self.dt, nx, ny, nz, *self.h, self.scheme)
+                # the fill's adjoint follows each step (lam's ghosts stay
+                # zero), so the last one is that of phi0's fill
+                D.passive_advect_adjoint_step(self.u, self.v, self.w, seg[n - n0], lam, lam2, self.au, self.av,
+                                              self.aw, self.dt, *self.h, self.scheme, self.phi_bc)
                 lam, lam2 = lam2, lam
-        D.bc_adjoint_nocorners(lam, self.phi_bc)  # the initial fill of phi0
         grad_phi0 = lam.interior().clone()
         self._project_adjoint()
         grads = []

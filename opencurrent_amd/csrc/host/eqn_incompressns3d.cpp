@@ -421,8 +421,11 @@ bool Eqn_ScalarAdvection3D<T>::advance_one_step(double dt) {
     return false;
   }
   check_ok(_advection.solve());
-  check_ok(phi.linear_combination((T)1, phi, (T)dt, deriv_phidt));
-  check_ok(apply_3d_boundary_conditions_level1_nocorners(phi, bc, hx(), hy(), hz()));
+  const ocu_grid3d p = phi.desc(), d = deriv_phidt.desc();
+  const ocu_bc_set b = to_c_bc(bc);
+  check_ok(ocu_status_ok(ocu_grid_lincomb_fill(&p, 1.0, &p, (double)(T)dt, &d, &b, hx(), hy(), hz(),
+                                               ThreadManager::get_compute_stream()),
+                         "Eqn_ScalarAdvection3D::advance_one_step"));
   return !any_error();
 }
 

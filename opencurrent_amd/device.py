@@ -211,6 +211,12 @@ def grid_lincomb(r, a1, g1, a2=0.0, g2=None):
                "grid_lincomb")
 
 
+def grid_lincomb_fill(r, a1, g1, a2, g2, bc, hx, hy, hz):
+    """r = a1*g1 + a2*g2, then the no-corner ghost fill of r"""
+    _lib.check(_lib.hip().ocu_grid_lincomb_fill(r.ptr(), a1, g1.ptr(), a2, g2.ptr(), C.byref(bc), hx, hy, hz, None),
+               "grid_lincomb_fill")
+
+
 def grid_copy(dst, src):
     _lib.check(_lib.hip().ocu_grid_copy(dst.ptr(), src.ptr(), None), "grid_copy")
 
@@ -258,6 +264,19 @@ def passive_advect_adjoint(u, v, w, phi, lam, lam_out, au, av, aw, scale, nx, ny
     _lib.check(_lib.hip().ocu_passive_advect_adjoint(u.ptr(), v.ptr(), w.ptr(), phi.ptr(), lam.ptr(), lam_out.ptr(),
                                                      au.ptr(), av.ptr(), aw.ptr(), scale, nx, ny, nz, hx, hy, hz,
                                                      scheme, None), "passive_advect_adjoint")
+
+
+def passive_advect_step(u, v, w, phi, phi_out, dphi, dt, hx, hy, hz, scheme, bc):
+    """phi_out = fill(phi + dt * A(u, phi)); dphi is scratch"""
+    _lib.check(_lib.hip().ocu_passive_advect_step(u.ptr(), v.ptr(), w.ptr(), phi.ptr(), phi_out.ptr(), dphi.ptr(), dt,
+                                                  hx, hy, hz, scheme, C.byref(bc), None), "passive_advect_step")
+
+
+def passive_advect_adjoint_step(u, v, w, phi, lam, lam_out, au, av, aw, scale, hx, hy, hz, scheme, bc):
+    """passive_advect_adjoint, then bc_adjoint_nocorners on lam_out; lam's ghost layer is zero"""
+    _lib.check(_lib.hip().ocu_passive_advect_adjoint_step(u.ptr(), v.ptr(), w.ptr(), phi.ptr(), lam.ptr(),
+                                                          lam_out.ptr(), au.ptr(), av.ptr(), aw.ptr(), scale, hx, hy,
+                                                          hz, scheme, C.byref(bc), None), "passive_advect_adjoint_step")
 
 
 def bc_adjoint_nocorners(g, bc):
