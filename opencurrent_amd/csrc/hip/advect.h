@@ -143,12 +143,11 @@ __device__ __forceinline__ Far2 far2(int c, int n, int top, int64_t s, bool per)
   f.hi = (c + 2 <= top ? (int64_t)2 : (int64_t)(whi - c)) * s;
   return f;
 }
-// far2 for a cell whose samples do not wrap (not within two cells of a
-// periodic boundary): the same flags and offsets with the offsets constant
-__device__ __forceinline__ Far2 far2_nowrap(int c, int top, int64_t s) {
+// far2 where the accessor wraps by itself: the same flags, the offsets constant
+__device__ __forceinline__ Far2 far2_nowrap(int c, int top, int64_t s, bool per) {
   Far2 f;
-  f.hlo = c >= 1;
-  f.hhi = c + 2 <= top;
+  f.hlo = c >= 1 || per;
+  f.hhi = c + 2 <= top || per;
   f.lo = -2 * s;
   f.hi = 2 * s;
   return f;
@@ -165,7 +164,7 @@ __device__ __forceinline__ T dflux2(const A &X, int64_t s, const Far2 &f, T vh, 
 
 // self-advection with second-order upwind face values: the face velocities
 // and flux terms of self_advect_at.  WRAP: far samples may wrap around a
-// periodic axis (far2); otherwise the caller guarantees they do not.
+// periodic axis (far2); otherwise the accessor does that by itself.
 template <bool WRAP, typename T, typename A>
 __device__ __forceinline__ void self_advect_up2_at(const A &U, const A &V, const A &W, int64_t xs, int64_t ys,
                                                    Inv<T> ih, int i, int j, int k, int nx, int ny, int nz, int pmask,
@@ -173,7 +172,7 @@ __device__ __forceinline__ void self_advect_up2_at(const A &U, const A &V, const
   const int64_t pi = xs, pj = ys, pk = 1, mi = -xs, mj = -ys, mk = -1;
   const bool px = pmask & 1, py = pmask & 2, pz = pmask & 4;
   auto far = [&](int c, int n, int top, int64_t s, bool per) {
-    return WRAP ? far2(c, n, top, s, per) : far2_nowrap(c, top, s);
+    return WRAP ? far2(c, n, top, s, per) : far2_nowrap(c, top, s, per);
   };
   // tangential (t) and normal (n) ghost extents per axis
   const Far2 fxt = far(i, nx, nx, xs, px), fxn = far(i, nx, nx + 1, xs, px);
@@ -212,7 +211,7 @@ __device__ __forceinline__ T passive_advect_up2_at(const A &u, const A &v, const
                                                    int64_t ys, Inv<T> ih, int i, int j, int k, int nx, int ny, int nz,
                                                    int pmask) {
   auto far = [&](int c, int n, int top, int64_t s, bool per) {
-    return WRAP ? far2(c, n, top, s, per) : far2_nowrap(c, top, s);
+    return WRAP ? far2(c, n, top, s, per) : far2_nowrap(c, top, s, per);
   };
   const T du = dflux2(phi, xs, far(i, nx, nx, xs, pmask & 1), u(xs), u(0));
   const T dv = dflux2(phi, ys, far(j, ny, ny, ys, pmask & 2), v(ys), v(0));

@@ -19,17 +19,13 @@
 //     grids being zero outside the cells their operators write;
 //   - with the interior-only combination they keep the old value;
 //   - T's face ghosts take the no-corner fill of the new interior value
-//     they derive from (recomputed by the ghost's own thread).
+//     they derive from (the interior is written first).
 #include "advect.h"
+#include "faces.h"
 
 using namespace ocu_hip;
 
 namespace {
-
-struct TFace {
-  int type;
-  float value;
-};
 
 template <typename T>
 struct NSStep {
@@ -39,7 +35,7 @@ struct NSStep {
   const T *lu, *lv, *lw, *lt;   // AB2: the last step's tendencies (read)
   Inv<T> ih, ih2;
   T nu, kappa, tcoef, a_dt, a_ab, th[3];
-  TFace tf[6];  // xpos, xneg, ypos, yneg, zpos, zneg
+  Faces tf;
   int64_t xs, ys, shift, vnbr;
   int pre, nx, ny, nz, gx, gy, gz, pnx, pny, pnz;
   int scheme, fper, tper, vaxis, flat, keep, use_last, visc, tdiff;
@@ -59,119 +55,44 @@ __device__ __forceinline__ T untouched(const NSStep<T> &s, int grid, T old) {
   return ((s.flat >> grid) & 1) ? combine(s, old, (T)0, (T)0) : old;
 }
 
-// T's tendency at interior cell c (offset from cell (0,0,0)): passive
-// advection, then + kappa*lap(T)
-template <typename T>
-__device__ __forceinline__ T temp_tendency(const NSStep<T> &s, int64_t c, int i, int j, int k) {
-  const T *U = s.u + s.shift, *V = s.v + s.shift, *W = s.w + s.shift, *Tt = s.t + s.shift;
-  T d = s.scheme == OCU_IT_SECOND_ORDER_UPWIND
-            ? passive_advect_up2_cell(U, V, W, Tt, c, s.xs, s.ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.tper)
-            : passive_advect_cell(U, V, W, Tt, c, s.xs, s.ys, s.ih, s.scheme);
-  if (s.tdiff) d = d + s.kappa * laplacian_cell(Tt, c, s.xs, s.ys, s.ih2);
-  return d;
-}
-
-// no-corner ghost value (grid3dboundary.cu:28-119): Dirichlet in double
-// (`-phi + 2.0 * (T)value`), Neumann phi -/+ h*value in T, periodic a copy
-template <typename T>
-__device__ __forceinline__ T nocorner_xform(const TFace &f, bool neg, T h, T a) {
-  if (f.type == OCU_BC_DIRICHELET) return (T)(-(double)a + 2.0 * (double)(T)f.value);
-  if (f.type == OCU_BC_NEUMANN) return neg ? a - h * (T)f.value : a + h * (T)f.value;
-  return a;
-}
-
-__device__ __forceinline__ bool tf_writes(const TFace &f) {
-  return f.type == OCU_BC_PERIODIC || f.type == OCU_BC_DIRICHELET || f.type == OCU_BC_NEUMANN;
-}
-
 // One element (ip, jp, kp) of the padded box (indices from the box corner,
-// ghosts included): the new value of each grid there.
+// ghosts included) outside T's interior: the new value of each grid there.
 template <typename T>
 __device__ __forceinline__ void ns_element(const NSStep<T> &s, int ip, int jp, int kp) {
   const int i = ip - s.gx, j = jp - s.gy, k = kp - s.gz;
   const int64_t e = (int64_t)s.pre + ((int64_t)ip * s.pny + jp) * s.pnz + kp;  // element of the allocation
-  const int64_t c = e - s.shift;                                               // offset from cell (0,0,0)
-  const T *U = s.u + s.shift, *V = s.v + s.shift, *W = s.w + s.shift, *Tt = s.t + s.shift;
-
   const bool ci = i >= 0 && i < s.nx, cj = j >= 0 && j < s.ny, ck = k >= 0 && k < s.nz;
-  // interiors of the four grids: u (nx+1,ny,nz), v (nx,ny+1,nz), w (nx,ny,nz+1), T (nx,ny,nz)
-  const bool in_u = i >= 0 && i <= s.nx && cj && ck;
-  const bool in_v = ci && j >= 0 && j <= s.ny && ck;
-  const bool in_w = ci && cj && k >= 0 && k <= s.nz;
-  const bool in_t = ci && cj && ck;
-
-  T du = 0, dv = 0, dw = 0;
-  if (in_t) {  // advection covers the cell box
-    if (s.scheme == OCU_IT_SECOND_ORDER_UPWIND)
-      self_advect_up2_cell(U, V, W, c, s.xs, s.ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.fper, du, dv, dw);
-    else
-      self_advect_cell(U, V, W, c, s.xs, s.ys, s.ih, s.scheme, du, dv, dw);
-  }
-  if (s.visc) {
-    if (in_u) du = du + s.nu * laplacian_cell(U, c, s.xs, s.ys, s.ih2);
-    if (in_v) dv = dv + s.nu * laplacian_cell(V, c, s.xs, s.ys, s.ih2);
-    if (in_w) dw = dw + s.nu * laplacian_cell(W, c, s.xs, s.ys, s.ih2);
-  }
-  if (in_t) {  // the thermal force covers the cell box of the vertical component
-    const T f = thermal_cell(Tt, c, s.vnbr, s.tcoef);
-    if (s.vaxis == 0) du = du + f;
-    else if (s.vaxis == 1) dv = dv + f;
-    else dw = dw + f;
-  }
-
-  if (in_u) {
-    s.un[e] = combine(s, U[c], du, s.use_last ? s.lu[e] : (T)0);
-    if (s.keep) s.du[e] = du;
-  } else {
-    s.un[e] = untouched(s, 0, U[c]);
-  }
-  if (in_v) {
-    s.vn[e] = combine(s, V[c], dv, s.use_last ? s.lv[e] : (T)0);
-    if (s.keep) s.dv[e] = dv;
-  } else {
-    s.vn[e] = untouched(s, 1, V[c]);
-  }
-  if (in_w) {
-    s.wn[e] = combine(s, W[c], dw, s.use_last ? s.lw[e] : (T)0);
-    if (s.keep) s.dw[e] = dw;
-  } else {
-    s.wn[e] = untouched(s, 2, W[c]);
-  }
-
-  if (in_t) {
-    const T dt = temp_tendency(s, c, i, j, k);
-    s.tn[e] = combine(s, Tt[c], dt, s.use_last ? s.lt[e] : (T)0);
-    if (s.keep) s.dtt[e] = dt;
-    return;
-  }
-  // a face ghost of T (one index at -1 or n, the others interior) that the
-  // no-corner fill writes: the fill of the new value of its source cell
-  const bool gx_ = (i == -1 || i == s.nx) && cj && ck, gy_ = ci && (j == -1 || j == s.ny) && ck,
-             gz_ = ci && cj && (k == -1 || k == s.nz);
-  // (the face and spacing picked by selects: an indexed read of the
-  // parameter arrays would copy them to scratch memory)
-  int si = i, sj = j, sk = k;
-  bool neg = false, has = false;
-  TFace f{OCU_BC_NONE, 0.f};
+  // the faces past the last cells: advection and the thermal force cover the
+  // cell box only
+  auto face = [&](const T *old, T *out, T *d, const T *last, int grid, bool in) {
+    if (!in) {
+      out[e] = untouched(s, grid, old[e]);
+      return;
+    }
+    T t = 0;
+    if (s.visc) t = t + s.nu * laplacian_cell(old, e, s.xs, s.ys, s.ih2);
+    out[e] = combine(s, old[e], t, s.use_last ? last[e] : (T)0);
+    if (s.keep) d[e] = t;
+  };
+  face(s.u, s.un, s.du, s.lu, 0, i == s.nx && cj && ck);
+  face(s.v, s.vn, s.dv, s.lv, 1, ci && j == s.ny && ck);
+  face(s.w, s.wn, s.dw, s.lw, 2, ci && cj && k == s.nz);
+  // a face ghost of T that the no-corner fill writes takes the fill of its
+  // source cell's new value, which k_ns_march has stored
+  Face f{OCU_BC_NONE, 0.f, 0.f};
+  bool neg = false;
   T h = 0;
-  if (gx_) {
-    neg = i < 0, f = neg ? s.tf[1] : s.tf[0], h = s.th[0], has = true;
-    si = f.type == OCU_BC_PERIODIC ? (neg ? s.nx - 1 : 0) : (neg ? 0 : s.nx - 1);
-  } else if (gy_) {
-    neg = j < 0, f = neg ? s.tf[3] : s.tf[2], h = s.th[1], has = true;
-    sj = f.type == OCU_BC_PERIODIC ? (neg ? s.ny - 1 : 0) : (neg ? 0 : s.ny - 1);
-  } else if (gz_) {
-    neg = k < 0, f = neg ? s.tf[5] : s.tf[4], h = s.th[2], has = true;
-    sk = f.type == OCU_BC_PERIODIC ? (neg ? s.nz - 1 : 0) : (neg ? 0 : s.nz - 1);
-  }
-  if (has && tf_writes(f)) {
-    const int64_t cs = (int64_t)si * s.xs + (int64_t)sj * s.ys + sk;
-    const T dt = temp_tendency(s, cs, si, sj, sk);
-    const T tnew = combine(s, Tt[cs], dt, s.use_last ? s.lt[cs + s.shift] : (T)0);
-    s.tn[e] = nocorner_xform(f, neg, h, tnew);
-  } else {
-    s.tn[e] = untouched(s, 3, Tt[c]);
-  }
+  int64_t from = 0;
+  auto ghost = [&](const Face &lo, const Face &hi, int c, int n, T hh, int64_t st) {
+    neg = c < 0;
+    f = neg ? lo : hi;
+    h = hh;
+    from = (int64_t)(src_index(f, neg, n) - c) * st;
+  };
+  if ((i == -1 || i == s.nx) && cj && ck) ghost(s.tf.xneg, s.tf.xpos, i, s.nx, s.th[0], s.xs);
+  else if (ci && (j == -1 || j == s.ny) && ck) ghost(s.tf.yneg, s.tf.ypos, j, s.ny, s.th[1], s.ys);
+  else if (ci && cj && (k == -1 || k == s.nz)) ghost(s.tf.zneg, s.tf.zpos, k, s.nz, s.th[2], 1);
+  s.tn[e] = writes(f) ? xform<T, true>(f, neg, h, s.tn[e + from]) : untouched(s, 3, s.t[e]);
 }
 
 // the pre-padding before the padded box: untouched elements
@@ -183,46 +104,39 @@ __device__ __forceinline__ void ns_prepad(const NSStep<T> &s, int64_t e) {
   s.tn[e] = untouched(s, 3, s.t[e]);
 }
 
-// The interior core is the box [bx, nx-bx) x [by, ny-by) x [bz, nz-bz) of
-// T's interior (a band of b = 2 cells is left out along a periodic axis when
-// second-order upwind samples would wrap around it); k_ns_march takes the
-// core.  Every other element - the bands, the u, v and w faces at i = nx,
-// j = ny and k = nz, the ghost layers, the padding - goes here, one thread
-// each, after the pre-padding: the planes outside the core's x range (count
-// na), then the rows outside its y range of the core's planes (nb), then the
-// row ends outside its z range of the core's rows (nc).
-struct Core {
-  int bx, by, bz;
-};
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_ns_shell(NSStep<T> s, Core b, int64_t na, int64_t nb, int64_t nc) {
-  int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (q < s.pre) {
+// k_ns_march takes T's interior.  Every other element - the u, v and w faces
+// at i = nx, j = ny and k = nz, the ghost layers, the padding - goes here, one
+// thread each, after the pre-padding: the planes outside the interior's x
+// range (count na), then the rows outside its y range (nb), then the row ends
+// (nc).  I: the type of the element count (a thread's divisions take longer
+// than its copies in 64 bits).  Bound by the row ends, 16 elements of each row
+// of eight grids.
+template <typename T, typename I>
+__global__ __launch_bounds__(256) void k_ns_shell(NSStep<T> s, I na, I nb, I nc) {
+  I q = (I)blockIdx.x * 256 + threadIdx.x;
+  if (q < (I)s.pre) {
     ns_prepad(s, q);
     return;
   }
   q -= s.pre;
-  const int cx = s.nx - 2 * b.bx, cy = s.ny - 2 * b.by, cz = s.nz - 2 * b.bz;  // core extents
-  const int lx = s.gx + b.bx, ly = s.gy + b.by, lz = s.gz + b.bz;             // its low corner (box indices)
   int ip, jp, kp;
   if (q < na) {
-    const int64_t plane = (int64_t)s.pny * s.pnz, pl = q / plane, r = q % plane;
-    ip = pl < lx ? (int)pl : (int)pl + cx;
+    const I plane = (I)s.pny * s.pnz, pl = q / plane, r = q % plane;
+    ip = (int)pl < s.gx ? (int)pl : (int)pl + s.nx;
     jp = (int)(r / s.pnz);
     kp = (int)(r % s.pnz);
   } else if ((q -= na) < nb) {
-    const int64_t per = (int64_t)(s.pny - cy) * s.pnz, pl = q / per, r = q % per;
+    const I per = (I)(s.pny - s.ny) * s.pnz, pl = q / per, r = q % per;
     const int rr = (int)(r / s.pnz);
-    ip = (int)pl + lx;
-    jp = rr < ly ? rr : rr + cy;
+    ip = (int)pl + s.gx;
+    jp = rr < s.gy ? rr : rr + s.ny;
     kp = (int)(r % s.pnz);
   } else if ((q -= nb) < nc) {
-    const int per = s.pnz - cz, t = (int)(q % per);
-    const int64_t rowi = q / per;
-    ip = (int)(rowi / cy) + lx;
-    jp = (int)(rowi % cy) + ly;
-    kp = t < lz ? t : t + cz;
+    const int per = s.pnz - s.nz, t = (int)(q % per);
+    const I rowi = q / per;
+    ip = (int)(rowi / s.ny) + s.gx;
+    jp = (int)(rowi % s.ny) + s.gy;
+    kp = t < s.gz ? t : t + s.nz;
   } else {
     return;
   }
@@ -230,36 +144,59 @@ __global__ __launch_bounds__(256) void k_ns_shell(NSStep<T> s, Core b, int64_t n
 }
 
 // ------------------------------------------------------------------------
-// the interior core, marching along x through an LDS window
+// T's interior, marching along x
 // ------------------------------------------------------------------------
 //
-// A block owns a tile of MTJ rows x MTK cells (j, k) of T's interior (its
-// cells in the core) and an x-chunk of planes.  It keeps a window of planes p-2..p+2 of u, v, w and T
-// in LDS, each plane with a two-cell halo in j and k (every sample the
-// cell functions read: second-order upwind reaches two cells, the
-// self-advection velocities one diagonal), in six slots, so the plane
-// loading for p+1 goes to the slot no thread reads in plane p and one
-// barrier per plane orders the accesses.  The cell functions read the
-// window through WAt, whose offsets use a virtual x stride of 2^20 elements
-// (no sample of a core cell wraps around a periodic axis).  Each cell's
-// tendencies and new values are those of ns_element, in the same order.
-constexpr int MTK = 64, MTJ = 8, MWK = MTK + 4, MWJ = MTJ + 4, MPLANE = MWJ * MWK, MSLOTS = 6;
-constexpr int MXSH = 20;
+// A block owns a tile of MJ rows x 64 cells (j, k) of T's interior and a chunk
+// of planes.  A thread keeps its own column's u, v,
+// w, T of planes p-2..p+2 in registers and loads those of p+3; off the column
+// the cell functions read u at p and p+1, v and w at p-1 and p, and T at p
+// (second-order upwind reaches two cells along each axis but stays on it, the
+// self-advection velocities one diagonal), so the LDS holds only those planes
+// with a halo of R cells in j and k, and one more of each field being
+// written: 3 + 3 + 3 + 2.  That leaves room for 16 waves a CU in FP64 where
+// planes p-2..p+2 of all four fields left it for 8, and half the LDS reads.
+// The step, this kernel and the shell: 512x512x256 FP64 first-order upwind
+// 1648 -> 1090 us, 128^3 FP64 second-order upwind 95 -> 73 us, 128^3 FP32 37 ->
+// 28 and 55 -> 44 us; the traffic at the copy rate is 830, 26 and 13.
+// One barrier per plane orders the accesses: what plane p writes no thread
+// reads before plane p + 1.  A place two beyond the box is only ever the far
+// sample of second-order upwind, which wraps on a periodic axis: it is loaded
+// from where it wraps to, so the cells there are like all others.
+constexpr int MTK = 64;
+constexpr int MXSH = 20;  // the offsets' x stride is 2^20: no plane comes near it
 constexpr int64_t MXS = (int64_t)1 << MXSH;
-constexpr int MLOADS = (MPLANE + MTK * MTJ - 1) / (MTK * MTJ);  // window elements per thread and plane
 
+template <int R, int MJ>
+struct Win {
+  static constexpr int WK = MTK + 2 * R, WJ = MJ + 2 * R, PL = WJ * WK, HALO = PL - MTK * MJ;
+  // slots: u 0..2, v 3..5, w 6..8, T 9..10
+  static constexpr int SLOTS = 11;
+  static_assert(HALO <= MTK * MJ, "one halo cell per thread at most");
+};
+
+// A coordinate of a field's array along an axis of n cells with samples up to
+// -1 and top (far2): beyond them it wraps, or (no cell reads it) is the edge.
+__device__ __forceinline__ int wrapped(int q, int n, int top, bool per) {
+  if (q >= -1 && q <= top) return q;
+  return per ? ((q % n) + n) % n : q < 0 ? -1 : top;
+}
+
+// One field around a cell: planes p-2..p+2 of its column in registers, the
+// cell's place in the LDS planes p-1 (v, w), p and p+1 (u).  Every offset is
+// a constant, so one of them remains.
 template <typename T>
-struct WAt {
-  const T *base;               // this field's slot 0
-  int cell;                    // the cell within a window plane
-  int sm2, sm1, s0, sp1, sp2;  // element offsets of the slots of planes p-2..p+2
+struct Col {
+  T m2, m1, c, p1, p2;
+  const T *lm, *l0, *lp;
   __device__ __forceinline__ T operator()(int64_t o) const {
-    const int di = (int)((o + (MXS >> 1)) >> MXSH);
-    const int r = (int)(o - ((int64_t)di << MXSH));
-    // a chain of selects, not an array: constant offsets fold to one slot,
-    // and a computed one keeps the slots in registers
-    const int sl = di == -2 ? sm2 : di == -1 ? sm1 : di == 0 ? s0 : di == 1 ? sp1 : sp2;
-    return base[sl + cell + r];
+    if (o == 0) return c;
+    if (o == MXS) return p1;
+    if (o == -MXS) return m1;
+    if (o == 2 * MXS) return p2;
+    if (o == -2 * MXS) return m2;
+    const int di = (int)((o + (MXS >> 1)) >> MXSH), r = (int)(o - ((int64_t)di << MXSH));
+    return (di < 0 ? lm : di > 0 ? lp : l0)[r];
   }
 };
 
@@ -268,38 +205,38 @@ struct Tend {
   T du, dv, dw, dt;
 };
 
-// the tendencies of interior cell (i, j, k) through accessors A (window or
-// global): the sequence of ns_element for a cell of T's interior (returned
-// by value, so that the two callers' results stay in registers)
-template <bool WRAP, typename T, typename A>
-__device__ __forceinline__ Tend<T> ns_tendencies(const NSStep<T> &s, const A &U, const A &V, const A &W, const A &Tt,
-                                                 int64_t xs, int64_t ys, int64_t vnbr, int i, int j, int k) {
+// the tendencies of interior cell (i, j, k): the sequence of ns_element for a
+// cell of T's interior (returned by value, so that they stay in registers)
+template <int SCHEME, typename T>
+__device__ __forceinline__ Tend<T> ns_tendencies(const NSStep<T> &s, const Col<T> &U, const Col<T> &V, const Col<T> &W,
+                                                 const Col<T> &Tt, int64_t ys, int i, int j, int k) {
+  constexpr int64_t xs = MXS;
   T du, dv, dw, dt;
-  if (s.scheme == OCU_IT_SECOND_ORDER_UPWIND)
-    self_advect_up2_at<WRAP, T>(U, V, W, xs, ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.fper, du, dv, dw);
+  if (SCHEME == OCU_IT_SECOND_ORDER_UPWIND)
+    self_advect_up2_at<false, T>(U, V, W, xs, ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.fper, du, dv, dw);
   else
-    self_advect_at<T>(U, V, W, xs, ys, s.ih, s.scheme, du, dv, dw);
+    self_advect_at<T>(U, V, W, xs, ys, s.ih, SCHEME, du, dv, dw);
   if (s.visc) {
     du = du + s.nu * laplacian_at<T>(U, xs, ys, s.ih2);
     dv = dv + s.nu * laplacian_at<T>(V, xs, ys, s.ih2);
     dw = dw + s.nu * laplacian_at<T>(W, xs, ys, s.ih2);
   }
-  const T f = thermal_at<T>(Tt, vnbr, s.tcoef);
-  if (s.vaxis == 0) du = du + f;
-  else if (s.vaxis == 1) dv = dv + f;
-  else dw = dw + f;
-  dt = s.scheme == OCU_IT_SECOND_ORDER_UPWIND
-           ? passive_advect_up2_at<WRAP, T>(U, V, W, Tt, xs, ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.tper)
-           : passive_advect_at<T>(U, V, W, Tt, xs, ys, s.ih, s.scheme);
+  if (s.vaxis == 0) du = du + thermal_at<T>(Tt, xs, s.tcoef);
+  else if (s.vaxis == 1) dv = dv + thermal_at<T>(Tt, ys, s.tcoef);
+  else dw = dw + thermal_at<T>(Tt, (int64_t)1, s.tcoef);
+  dt = SCHEME == OCU_IT_SECOND_ORDER_UPWIND
+           ? passive_advect_up2_at<false, T>(U, V, W, Tt, xs, ys, s.ih, i, j, k, s.nx, s.ny, s.nz, s.tper)
+           : passive_advect_at<T>(U, V, W, Tt, xs, ys, s.ih, SCHEME);
   if (s.tdiff) dt = dt + s.kappa * laplacian_at<T>(Tt, xs, ys, s.ih2);
   return Tend<T>{du, dv, dw, dt};
 }
 
-template <typename T>
-__global__ __launch_bounds__(MTK *MTJ) void k_ns_march(NSStep<T> s, Core b, int tiles_k, int tiles_j, int ichunk,
-                                                       int ntiles) {
+template <typename T, int SCHEME, int R, int MJ>
+__global__ __launch_bounds__(MTK *MJ) void k_ns_march(NSStep<T> s, int tiles_k, int tiles_j, int ichunk,
+                                                      int ntiles) {
+  typedef Win<R, MJ> W;
   extern __shared__ unsigned char ns_smem[];
-  T *win = reinterpret_cast<T *>(ns_smem);  // [4 fields][MSLOTS][MPLANE]
+  T *win = reinterpret_cast<T *>(ns_smem);  // [SLOTS][PL]
   // blocks are dealt round-robin to the 8 XCDs: a contiguous run of tiles
   // per XCD
   const int per = gridDim.x / 8;
@@ -307,72 +244,98 @@ __global__ __launch_bounds__(MTK *MTJ) void k_ns_march(NSStep<T> s, Core b, int 
   if (logical >= ntiles) return;  // uniform per block
   const int tk = logical % tiles_k, rem = logical / tiles_k, tj = rem % tiles_j, ti = rem / tiles_j;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * MTK + tx;
-  const int k0 = tk * MTK, j0 = tj * MTJ, i0 = ti * ichunk, i1 = min(s.nx, i0 + ichunk);
+  const int k0 = tk * MTK, j0 = tj * MJ, i0 = ti * ichunk, i1 = min(s.nx, i0 + ichunk);
   const int k = k0 + tx, j = j0 + ty;
-  const bool mine = k >= b.bz && k < s.nz - b.bz && j >= b.by && j < s.ny - b.by;
-  const T *src[4] = {s.u, s.v, s.w, s.t};
+  const bool mine = k < s.nz && j < s.ny;
+  const T *src[4] = {s.u + s.pre, s.v + s.pre, s.w + s.pre, s.t + s.pre};  // corner of the padded box
+  const int64_t plane = (int64_t)s.pny * s.pnz;
 
-  // element offsets (from element 0) of this thread's window positions in
-  // plane 0 (-1: outside the padded box in j or k)
-  int64_t wpos[MLOADS];
-#pragma unroll
-  for (int m = 0; m < MLOADS; m++) {
-    const int t = tid + m * MTK * MTJ;
-    const int wj = t / MWK, wk = t % MWK;
-    const int jp = j0 - 2 + wj + s.gy, kp = k0 - 2 + wk + s.gz;
-    wpos[m] = (t < MPLANE && jp >= 0 && jp < s.pny && kp >= 0 && kp < s.pnz)
-                  ? (int64_t)s.pre + (int64_t)jp * s.pnz + kp
-                  : (int64_t)-1;
+  // this thread's own place and its halo place in the window, and their
+  // elements in a plane of each field's padded box
+  const int cell = (ty + R) * W::WK + tx + R;
+  auto element = [&](int f, int wj, int wk) {
+    const int per_ = f == 3 ? s.tper : s.fper;
+    const int jj = wrapped(j0 - R + wj, s.ny, s.ny + (R == 2 && f == 1), R == 2 && (per_ & 2));
+    const int kk = wrapped(k0 - R + wk, s.nz, s.nz + (R == 2 && f == 2), R == 2 && (per_ & 4));
+    return (jj + s.gy) * s.pnz + kk + s.gz;
+  };
+  const bool has_halo = tid < W::HALO;
+  int hwj, hwk;  // rows above and below the tile, then the row ends
+  {
+    constexpr int FULL = 2 * R * W::WK;
+    if (tid < FULL) {
+      hwj = tid / W::WK, hwk = tid % W::WK;
+      if (hwj >= R) hwj += MJ;
+    } else {
+      const int q = tid - FULL, e = q % (2 * R);
+      hwj = R + min(q / (2 * R), MJ - 1), hwk = e < R ? e : e + MTK;
+    }
   }
-  auto slot = [](int q) { return ((q % MSLOTS) + MSLOTS) % MSLOTS; };
-  auto fetch = [&](int q, T (&v)[4][MLOADS]) {
-    const int ip = q + s.gx;
-    const bool in = ip >= 0 && ip < s.pnx;
+  const int hcell = hwj * W::WK + hwk;
+  int own_e[4], halo_e[4];
 #pragma unroll
-    for (int m = 0; m < MLOADS; m++) {
-      const bool ok = in && wpos[m] >= 0;
-      const int64_t e = wpos[m] + (int64_t)ip * s.pny * s.pnz;
-#pragma unroll
-      for (int f = 0; f < 4; f++) v[f][m] = ok ? src[f][e] : (T)0;
-    }
+  for (int f = 0; f < 4; f++) own_e[f] = element(f, ty + R, tx + R), halo_e[f] = element(f, hwj, hwk);
+  auto at = [&](int f, int q) {
+    const int ii = wrapped(q, s.nx, s.nx + (R == 2 && f == 0), R == 2 && ((f == 3 ? s.tper : s.fper) & 1));
+    return src[f] + (int64_t)(ii + s.gx) * plane;
   };
-  auto store = [&](int q, const T (&v)[4][MLOADS]) {
-    T *dst = win + slot(q) * MPLANE;
+  auto slot = [&](int f, int q) { return win + (f * 3 + (f == 3 ? q & 1 : (unsigned)(q + 3) % 3)) * W::PL; };
+
+  T m2[4], m1[4], c0[4], p1[4], p2[4], nx_[4], h[4];
 #pragma unroll
-    for (int m = 0; m < MLOADS; m++) {
-      const int t = tid + m * MTK * MTJ;
-      if (t < MPLANE) {
+  for (int f = 0; f < 4; f++) {
+    m2[f] = at(f, i0 - 2)[own_e[f]], m1[f] = at(f, i0 - 1)[own_e[f]], c0[f] = at(f, i0)[own_e[f]];
+    p1[f] = at(f, i0 + 1)[own_e[f]], p2[f] = at(f, i0 + 2)[own_e[f]];
+  }
+  T ha[4] = {}, hb[3] = {};  // halo: u, v, w, T at i0; u at i0 + 1, v and w at i0 - 1
 #pragma unroll
-        for (int f = 0; f < 4; f++) dst[f * MSLOTS * MPLANE + t] = v[f][m];
-      }
+  for (int f = 0; f < 4; f++) h[f] = (T)0;
+  if (has_halo) {
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      ha[f] = at(f, i0)[halo_e[f]];
+      if (f < 3) hb[f] = at(f, f == 0 ? i0 + 1 : i0 - 1)[halo_e[f]];
+      h[f] = at(f, f == 0 ? i0 + 2 : i0 + 1)[halo_e[f]];
     }
-  };
-  T v[4][MLOADS];
-  for (int q = i0 - 2; q <= i0 + 2; q++) {
-    fetch(q, v);
-    store(q, v);
+  }
+#pragma unroll
+  for (int f = 0; f < 4; f++) {
+    slot(f, i0)[cell] = c0[f];
+    if (f < 3) slot(f, f == 0 ? i0 + 1 : i0 - 1)[cell] = f == 0 ? p1[f] : m1[f];
+  }
+  if (has_halo) {
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      slot(f, i0)[hcell] = ha[f];
+      if (f < 3) slot(f, f == 0 ? i0 + 1 : i0 - 1)[hcell] = hb[f];
+    }
   }
   __syncthreads();
 
-  const int cell = (ty + 2) * MWK + tx + 2;
-  const int64_t xs = s.xs, ys = s.ys;
-  const int64_t vnbr_w = s.vaxis == 0 ? MXS : s.vaxis == 1 ? (int64_t)MWK : (int64_t)1;
   for (int p = i0; p < i1; p++) {
-    fetch(p + 3, v);  // in flight while plane p is computed
-    if (mine && p >= b.bx && p < s.nx - b.bx) {
-      const int64_t c = (int64_t)p * xs + (int64_t)j * ys + k;  // offset from cell (0,0,0)
-      const int sm2 = slot(p - 2) * MPLANE, sm1 = slot(p - 1) * MPLANE, s0 = slot(p) * MPLANE,
-                sp1 = slot(p + 1) * MPLANE, sp2 = slot(p + 2) * MPLANE;
-      auto acc = [&](int f) { return WAt<T>{win + f * MSLOTS * MPLANE, cell, sm2, sm1, s0, sp1, sp2}; };
-      const Tend<T> d = ns_tendencies<false, T>(s, acc(0), acc(1), acc(2), acc(3), MXS, (int64_t)MWK, vnbr_w, p, j, k);
-      const int64_t e = c + s.shift;
-      const T *olds = win + slot(p) * MPLANE + cell;
-      const T ou = olds[0], ov = olds[MSLOTS * MPLANE], ow = olds[2 * MSLOTS * MPLANE],
-              ot = olds[3 * MSLOTS * MPLANE];
-      s.un[e] = combine(s, ou, d.du, s.use_last ? s.lu[e] : (T)0);
-      s.vn[e] = combine(s, ov, d.dv, s.use_last ? s.lv[e] : (T)0);
-      s.wn[e] = combine(s, ow, d.dw, s.use_last ? s.lw[e] : (T)0);
-      s.tn[e] = combine(s, ot, d.dt, s.use_last ? s.lt[e] : (T)0);
+    // the planes that p + 1 reads: u at p+2; v, w, T at p+1
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      T *dst = slot(f, f == 0 ? p + 2 : p + 1);
+      dst[cell] = f == 0 ? p2[f] : p1[f];
+      if (has_halo) dst[hcell] = h[f];
+    }
+    // in flight while plane p is computed
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      nx_[f] = at(f, p + 3)[own_e[f]];
+      if (has_halo) h[f] = at(f, f == 0 ? p + 3 : p + 2)[halo_e[f]];
+    }
+    if (mine) {
+      const int64_t e = (int64_t)p * s.xs + (int64_t)j * s.ys + k + s.shift;
+      auto col = [&](int f) {
+        return Col<T>{m2[f], m1[f], c0[f], p1[f], p2[f], slot(f, p - 1) + cell, slot(f, p) + cell, slot(f, p + 1) + cell};
+      };
+      const Tend<T> d = ns_tendencies<SCHEME, T>(s, col(0), col(1), col(2), col(3), (int64_t)W::WK, p, j, k);
+      s.un[e] = combine(s, c0[0], d.du, s.use_last ? s.lu[e] : (T)0);
+      s.vn[e] = combine(s, c0[1], d.dv, s.use_last ? s.lv[e] : (T)0);
+      s.wn[e] = combine(s, c0[2], d.dw, s.use_last ? s.lw[e] : (T)0);
+      s.tn[e] = combine(s, c0[3], d.dt, s.use_last ? s.lt[e] : (T)0);
       if (s.keep) {
         s.du[e] = d.du;
         s.dv[e] = d.dv;
@@ -380,7 +343,8 @@ __global__ __launch_bounds__(MTK *MTJ) void k_ns_march(NSStep<T> s, Core b, int 
         s.dtt[e] = d.dt;
       }
     }
-    store(p + 3, v);
+#pragma unroll
+    for (int f = 0; f < 4; f++) m2[f] = m1[f], m1[f] = c0[f], c0[f] = p1[f], p1[f] = p2[f], p2[f] = nx_[f];
     __syncthreads();
   }
 }
@@ -398,6 +362,36 @@ int check_congruent(const ocu_grid3d *a, const ocu_grid3d *b, const char *what) 
 bool whole_allocation(const ocu_grid3d *g) {
   const int64_t interior = (int64_t)g->nx * g->ny * g->nz;
   return !((g->allocated - interior) / (float)g->allocated > .03f);
+}
+
+template <typename T, int SCHEME, int R, int MJ>
+int launch_march(const NSStep<T> &s, hipStream_t stream) {
+  const auto kernel = &k_ns_march<T, SCHEME, R, MJ>;
+  const int tiles_k = (s.nz + MTK - 1) / MTK, tiles_j = (s.ny + MJ - 1) / MJ;
+  const size_t lds = (size_t)Win<R, MJ>::SLOTS * Win<R, MJ>::PL * sizeof(T);
+  OCU_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds));
+  int dev = 0, cus = 256, per = 1;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+    cus = 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, MTK * MJ, lds) != hipSuccess || per < 1) per = 1;
+  // planes per block: the fewest rounds of resident blocks, each block
+  // loading four planes beyond its own
+  const int64_t slots = (int64_t)cus * per;
+  int ichunk = s.nx;
+  int64_t best = INT64_MAX;
+  for (int ic = 1;; ic = ic < 8 ? ic + 1 : ic * 2) {
+    const int c = min(ic, s.nx);  // the last candidate is the whole extent
+    const int64_t nb_ = (int64_t)tiles_k * tiles_j * ((s.nx + c - 1) / c);
+    const int64_t cost = ((nb_ + slots - 1) / slots) * (c + 4);
+    if (cost < best) best = cost, ichunk = c;
+    if (c == s.nx) break;
+  }
+  const int ntiles = tiles_k * tiles_j * ((s.nx + ichunk - 1) / ichunk);
+  const int nblocks = ((ntiles + 7) / 8) * 8;
+  kernel<<<nblocks, dim3(MTK, MJ), lds, stream>>>(s, tiles_k, tiles_j, ichunk, ntiles);
+  return OCU_OK;
 }
 
 template <typename T>
@@ -419,8 +413,7 @@ int launch_ns_step(const ocu_grid3d *const *in, const ocu_grid3d *const *out, co
   s.nu = (T)p->viscosity, s.kappa = (T)p->thermal_diffusion, s.tcoef = (T)p->thermal_coef;
   s.a_dt = (T)p->a_dt, s.a_ab = (T)p->a_ab;
   s.th[0] = (T)p->hx, s.th[1] = (T)p->hy, s.th[2] = (T)p->hz;
-  const ocu_bc *all[6] = {&tbc->xpos, &tbc->xneg, &tbc->ypos, &tbc->yneg, &tbc->zpos, &tbc->zneg};
-  for (int f = 0; f < 6; f++) s.tf[f] = TFace{all[f]->type, all[f]->value};
+  s.tf = faces(tbc);
   s.xs = (int64_t)g->pny * g->pnz, s.ys = g->pnz, s.shift = g->shift;
   const int vd = p->vertical_direction;
   s.vaxis = (vd & OCU_DIR_XAXIS_FLAG) ? 0 : (vd & OCU_DIR_YAXIS_FLAG) ? 1 : 2;
@@ -432,49 +425,28 @@ int launch_ns_step(const ocu_grid3d *const *in, const ocu_grid3d *const *out, co
   s.flat = 0;
   for (int q = 0; q < 4; q++) s.flat |= whole_allocation(in[q]) << q;
   s.visc = p->viscosity > 0, s.tdiff = p->thermal_diffusion > 0;
-  // the core: bands of two cells along the periodic axes whose second-order
-  // upwind samples wrap (flow or temperature)
-  Core b{0, 0, 0};
-  if (s.scheme == OCU_IT_SECOND_ORDER_UPWIND) {
-    const int per = s.fper | s.tper;
-    b.bx = (per & 1) ? 2 : 0, b.by = (per & 2) ? 2 : 0, b.bz = (per & 4) ? 2 : 0;
-  }
-  const bool core = s.nx > 2 * b.bx && s.ny > 2 * b.by && s.nz > 2 * b.bz;
-  if (!core) b = Core{(s.nx + 1) / 2, (s.ny + 1) / 2, (s.nz + 1) / 2};  // all to the shell
-  const int cx = max(s.nx - 2 * b.bx, 0), cy = max(s.ny - 2 * b.by, 0), cz = max(s.nz - 2 * b.bz, 0);
-  // the shell: everything outside the core
-  const int64_t na = (int64_t)(s.pnx - cx) * s.pny * s.pnz, nb = (int64_t)cx * (s.pny - cy) * s.pnz,
-                nc = (int64_t)cx * cy * (s.pnz - cz);
-  const int64_t nshell = s.pre + na + nb + nc;
-  k_ns_shell<T><<<(unsigned)((nshell + 255) / 256), 256, 0, stream>>>(s, b, na, nb, nc);
+  // the interior.  Rows per block: second-order upwind in FP64 needs 174
+  // registers, so 8 waves a CU (12 spill: 512x512x256 1.90 ms against 1.95, but
+  // 64^3 21.7 us against 19.2); the other schemes' 16 (14: 1.21 ms, 16: 1.09);
+  // FP32 has registers for several blocks of 8 a CU (256^3 195 us by 16 rows,
+  // 188 by 8)
+  constexpr int MJ = sizeof(T) == 8 ? 16 : 8;
+  int e;
+  if (s.scheme == OCU_IT_SECOND_ORDER_UPWIND) e = launch_march<T, OCU_IT_SECOND_ORDER_UPWIND, 2, 8>(s, stream);
+  else if (s.scheme == OCU_IT_SECOND_ORDER_CENTERED)
+    e = launch_march<T, OCU_IT_SECOND_ORDER_CENTERED, 1, MJ>(s, stream);
+  else e = launch_march<T, OCU_IT_FIRST_ORDER_UPWIND, 1, MJ>(s, stream);
+  if (e != OCU_OK) return e;
   OCU_HIP_TRY(hipGetLastError());
-  if (!core) return OCU_OK;
-  // the interior
-  const int tiles_k = (s.nz + MTK - 1) / MTK, tiles_j = (s.ny + MTJ - 1) / MTJ;
-  const size_t lds = (size_t)4 * MSLOTS * MPLANE * sizeof(T);
-  OCU_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ns_march<T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  int dev = 0, cus = 256, per = 1;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-    cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_ns_march<T>, MTK * MTJ, lds) != hipSuccess || per < 1)
-    per = 1;
-  // planes per block: the fewest rounds of resident blocks, each block
-  // loading four planes beyond its own
-  const int64_t slots = (int64_t)cus * per;
-  int ichunk = s.nx;
-  int64_t best = INT64_MAX;
-  for (int ic = 1;; ic = ic < 8 ? ic + 1 : ic * 2) {
-    const int c = min(ic, s.nx);  // the last candidate is the whole extent
-    const int64_t nb_ = (int64_t)tiles_k * tiles_j * ((s.nx + c - 1) / c);
-    const int64_t cost = ((nb_ + slots - 1) / slots) * (c + 4);
-    if (cost < best) best = cost, ichunk = c;
-    if (c == s.nx) break;
-  }
-  const int ntiles = tiles_k * tiles_j * ((s.nx + ichunk - 1) / ichunk);
-  const int nblocks = ((ntiles + 7) / 8) * 8;
-  k_ns_march<T><<<nblocks, dim3(MTK, MTJ), lds, stream>>>(s, b, tiles_k, tiles_j, ichunk, ntiles);
+  // the shell: everything outside T's interior
+  const int64_t na = (int64_t)(s.pnx - s.nx) * s.pny * s.pnz, nb = (int64_t)s.nx * (s.pny - s.ny) * s.pnz,
+                nc = (int64_t)s.nx * s.ny * (s.pnz - s.nz);
+  const int64_t nshell = s.pre + na + nb + nc;
+  const unsigned blocks = (unsigned)((nshell + 255) / 256);
+  if (nshell < INT32_MAX - 256)
+    k_ns_shell<T, unsigned><<<blocks, 256, 0, stream>>>(s, (unsigned)na, (unsigned)nb, (unsigned)nc);
+  else
+    k_ns_shell<T, int64_t><<<blocks, 256, 0, stream>>>(s, na, nb, nc);
   return OCU_OK;
 }
 
