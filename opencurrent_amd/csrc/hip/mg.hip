@@ -1982,9 +1982,18 @@ __global__ __launch_bounds__(BOT_THREADS) void k_mg_bottom(BotArgs<T, TC> args) 
 //   - the diagonals' reciprocals come from a 27-entry table (Recip).
 //   - a level of at most 64 blocks (8^3), or a coarsest level of at most 64
 //     cell pairs, is one wave's work: LDS operations of a wave are ordered, so
-//     it needs no barriers between colours.
+//     it needs no barriers between colours.  Each such level has a wave of its
+//     own, which works out its cells' places and reciprocals (some 1700
+//     cycles, more than two colours of the level take) while the level before
+//     runs, and a finished level is stored by the waves that the next one
+//     leaves idle.  Its prolongation is spread over the block, a thread per
+//     cell (2700 -> 1300 cycles).
+//   - what is known early is done while the first loads are in flight.
 // Measured against k_mg_bottom (one launch, launches included): 16^3 down to
-// 4^3 46.1 -> 21.6 us in FP64, 39.0 -> 18.3 mixed, 37.4 -> 17.7 in FP32;
+// 4^3 46.1 -> 18.2 us in FP64, 39.0 -> 15.1 mixed, 37.4 -> 15.0 in FP32 (21.6,
+// 18.3 and 17.7 with every thread setting up for every level); of the FP64
+// one's 40500 cycles the top level's colours take 10500, the second's 5800, the
+// coarsest 4000, the first loads 4400 and the last stores 4200;
 // 24x20x28 over 12x10x14 (84 coarsest iterations) in FP32 165 -> 62 us; the
 // coarsest level by itself (k_coarse_pairs against k_coarse) 22.4 -> 7.1 us
 // at 4^3 and 592 -> 43 us at 12x10x14.
@@ -2149,6 +2158,18 @@ __device__ __forceinline__ void blk_get(Blk<T> &s, const BlkLevel<T> &L, const i
   for (int e = 0; e < 8; e++) s.hb[e] = b_term(L.dc, B[s.own + e]);
 }
 
+// iters red-black iterations of a level of at most 64 blocks by one wave
+template <bool SIGN, typename T>
+__device__ __forceinline__ void blk_wave(Blk<T> &s, bool in, T *U, const typename DevCFor<T>::type &dc, int iters) {
+  const typename DevCFor<T>::type c = dc;
+  for (int it = 0; it < iters; it++) {
+    if (in) blk_colour<SIGN, 0>(s, U, c);
+    lds_sync(true);
+    if (in) blk_colour<SIGN, 1>(s, U, c);
+    lds_sync(true);
+  }
+}
+
 // iters red-black iterations; HELD: each thread's only block stays in s
 // (threads past the last block idle), else the blocks are reloaded for
 // every colour.  Ends with the block's threads in step.
@@ -2244,13 +2265,43 @@ __device__ __forceinline__ void blk_prolong(T (&u)[8], const T (&v)[3][3][3]) {
   }
 }
 
-// the ghost layer of a finished level to global memory: edges and corners
-// too, each from the cell it derives from, read through `at`
+// one cell of the prolongation (blk_prolong's operations and corner choice):
+// child e of coarse cell (ic,jc,kc), the coarse level read through `at`
 template <bool SIGN, typename T, typename AT>
-__device__ __forceinline__ void shell_store(const DGrid<T> &o, Mag mpy, Mag mz, const int *per, unsigned flip, AT at) {
+__device__ __forceinline__ T child_prolong(T u, int e, int ic, int jc, int kc, int nx, int ny, int nz, const int *per,
+                                           unsigned flip, AT at) {
+  const int c[3] = {ic, jc, kc}, n[3] = {nx, ny, nz}, d[3] = {e >> 2, (e >> 1) & 1, e & 1};
+  // the coarse cell beside it toward the child (or across x for the corner)
+  auto side = [&](int a, bool up, int &i, int &m) {
+    const bool edge = up ? c[a] == n[a] - 1 : c[a] == 0;
+    i = !edge ? c[a] + (up ? 1 : -1) : per[a] ? (up ? 0 : n[a] - 1) : c[a];
+    m = edge && ((flip >> (2 * a + !up)) & 1) ? (int)0x80000000 : 0;
+  };
+  int i[3], m[3], qi, qm;
+#pragma unroll
+  for (int a = 0; a < 3; a++) side(a, d[a], i[a], m[a]);
+  side(0, d[0] || e == 3, qi, qm);
+  auto get = [&](int x, int y, int z, int ms) {
+    const T t = at(x, y, z);
+    return SIGN ? flip_sign(t, ms) : t;
+  };
+  const T C = get(ic, jc, kc, 0);
+  const T X = get(i[0], jc, kc, m[0]), Y = get(ic, i[1], kc, m[1]), Z = get(ic, jc, i[2], m[2]);
+  const T XY = get(i[0], i[1], kc, m[0] ^ m[1]), XZ = get(i[0], jc, i[2], m[0] ^ m[2]),
+          YZ = get(ic, i[1], i[2], m[1] ^ m[2]);
+  const T XYZ = get(qi, i[1], i[2], qm ^ m[1] ^ m[2]);
+  return u + PW<T>::c0 * C + PW<T>::c1 * (X + Y + Z) + PW<T>::c2 * (XY + XZ + YZ) + PW<T>::c3 * XYZ;
+}
+
+// the ghost layer of a finished level to global memory: edges and corners
+// too, each from the cell it derives from, read through `at`, by the threads
+// id of cnt
+template <bool SIGN, typename T, typename AT>
+__device__ __forceinline__ void shell_store(const DGrid<T> &o, Mag mpy, Mag mz, const int *per, unsigned flip, int id,
+                                            int cnt, AT at) {
   const int nx = o.nx, ny = o.ny, nz = o.nz;
   const int nZ = (nx + 2) * (ny + 2), nY = (nx + 2) * nz, nX = ny * nz;
-  for (int t = threadIdx.x; t < 2 * (nZ + nY + nX); t += blockDim.x) {
+  for (int t = id; t < 2 * (nZ + nY + nX); t += cnt) {
     int i, j, k, q = t;
     if (q < 2 * nZ) {
       const int side = q >= nZ;
@@ -2302,9 +2353,11 @@ struct PairCell {
 template <bool SIGN, typename T>
 __device__ __forceinline__ void pair_cell(PairCell<T> &s, const PairGeom &g, const int *per, unsigned flip,
                                           const Recip<T> *tab, int col, int p) {
+  const bool in = p < g.n;
+  p = min(p, g.n - 1);  // threads past the last pair read its cells
   const int row = mdiv(p, g.mpair), m = p - row * g.npz, i = mdiv(row, g.my), j = row - i * g.ny;
   const int e = (i + j + col) & 1, k = 2 * m + e;
-  s.in = p < g.n && k < g.nz;
+  s.in = in && k < g.nz;
   s.own = col * g.n + p;
   const int oth = (1 - col) * g.n + p, sx = g.ny * g.npz, sy = g.npz;
   s.a[0] = k > 0 ? (e ? oth : oth - 1) : per[2] ? oth + g.npz - 1 : s.own;
@@ -2353,6 +2406,25 @@ __device__ __forceinline__ void pair_relax(PairCell<T> &s, T *U, const HostC<T> 
   }
   s.u = relax_host_q<P2>(c, s.u, v[0], v[1], v[2], v[3], v[4], v[5], s.hb, s.q);
   U[s.own] = s.u;
+}
+
+// iterations of relax_on_host on a thread's two cells by one wave
+template <bool SIGN, bool P2, typename T>
+__device__ __forceinline__ void pair_wave(PairCell<T> (&s)[2], T *U, const HostC<T> &cc, int iterations, int order) {
+  const HostC<T> c = cc;
+  for (int it = 0; it < iterations; it++) {
+    // uniform: the second half of the symmetric order starts black
+    if (color_of(order, it, iterations, 0) == 0) {
+      if (s[0].in) pair_relax<SIGN, P2>(s[0], U, c);
+      lds_sync(true);
+      if (s[1].in) pair_relax<SIGN, P2>(s[1], U, c);
+    } else {
+      if (s[1].in) pair_relax<SIGN, P2>(s[1], U, c);
+      lds_sync(true);
+      if (s[0].in) pair_relax<SIGN, P2>(s[0], U, c);
+    }
+    lds_sync(true);
+  }
 }
 
 // `iterations` iterations of relax_on_host on U (b in B), colours in
@@ -2414,13 +2486,13 @@ __device__ __forceinline__ void pair_solve(T *U, const T *B, const PairGeom &g, 
 // a finished coarsest level to global memory, ghosts included
 template <bool SIGN, typename TS, typename TC>
 __device__ __forceinline__ void pair_store(const DGrid<TS> &o, const TC *U, const PairGeom &g, const int *per,
-                                           unsigned flip) {
+                                           unsigned flip, int id, int cnt) {
   auto at = [&](int i, int j, int k) { return (TS)U[pair_elem(g, i, j, k)]; };
-  for (int t = threadIdx.x; t < g.nx * g.ny * g.nz; t += blockDim.x) {
+  for (int t = id; t < g.nx * g.ny * g.nz; t += cnt) {
     const int row = mdiv(t, g.mz), i = mdiv(row, g.my), j = row - i * g.ny, k = t - row * g.nz;
     o.at(i, j, k) = at(i, j, k);
   }
-  shell_store<SIGN>(o, g.mpy, g.mz, per, flip, at);
+  shell_store<SIGN>(o, g.mpy, g.mz, per, flip, id, cnt, at);
 }
 
 template <typename T>
@@ -2434,21 +2506,65 @@ __global__ __launch_bounds__(MAXT) void k_mg_bottom_blocks(BlkArgs<T, TC> args) 
   (void)args;
   const BlkArgs<T, TC> &A = *(const BlkArgs<T, TC> *)__builtin_amdgcn_kernarg_segment_ptr();
   extern __shared__ unsigned char smem[];
+  // registers for a block of the top level and one of a small level at a time
+  constexpr bool PREP = MAXT < BOT_THREADS;
+  // every line of the arguments on its way to the L2 at once: read when
+  // needed, each would be a trip to memory of its own
+  if (threadIdx.x * 64 < sizeof(BlkArgs<T, TC>))
+    (void)*(const volatile int *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() + threadIdx.x * 64);
   const int C = A.nlev - 1;
   const int per[3] = {A.per[0], A.per[1], A.per[2]};
   const unsigned flip = A.flip;
+  const int nw = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)),
+            lane = threadIdx.x & 63;
   auto U = [&](int l) { return (T *)(smem + A.L[l].uoff); };
   auto B = [&](int l) { return (T *)(smem + A.L[l].boff); };
   auto tab = [&](int l) { return (const Recip<T> *)(smem + A.L[l].toff); };
   TC *const uc = (TC *)(smem + A.cuoff), *const bc = (TC *)(smem + A.cboff);
   const Recip<TC> *const ctab = (const Recip<TC> *)(smem + A.ctoff);
 
-  // the top level's cells, every global load of a block in flight at once
+  // a small level is the work of one wave, another one for each level
+  auto small = [&](int l) { return PREP && l > 0 && l < C && nw > 1 && A.L[l].nb <= 64; };
+  auto mine = [&](int l) { return wave == l % nw; };
+  int fs = 0;  // the first small level: those below it are small too
+  while (fs < C && !small(fs)) fs++;
+  // the top level is the only large one and each thread has at most one block
+  // of it, which it keeps
+  const bool held0 = PREP && fs <= 1 && A.L[0].nb <= (int)blockDim.x;
+  auto places = [&](Blk<T> &k, int l, int blk) {
+    const BlkLevel<T> &L = A.L[l];
+    blk = min(blk, L.nb - 1);  // threads past the last block read its cells
+    int ic, jc, kc;
+    blk_coords(L, blk, ic, jc, kc);
+    blk_faces<SIGN>(k, L, per, flip, blk, ic, jc, kc);
+  };
+  auto recips = [&](Blk<T> &k, int l, int blk) {
+    const BlkLevel<T> &L = A.L[l];
+    int ic, jc, kc;
+    blk_coords(L, min(blk, L.nb - 1), ic, jc, kc);
+    blk_recips(k, L, tab(l), ic, jc, kc);
+  };
+  auto set_up = [&](Blk<T> &k, int l, int blk) { places(k, l, blk), recips(k, l, blk); };
+  auto cells = [&](Blk<T> &k, int l) {
+    const T *const u = U(l), *const b = B(l);
+#pragma unroll
+    for (int e = 0; e < 8; e++) k.u[e] = u[k.own + e], k.hb[e] = b_term(A.L[l].dc, b[k.own + e]);
+  };
+  auto set_up_pairs = [&](PairCell<TC> (&pc)[2]) {
+    pair_cell<SIGN>(pc[0], A.cg, per, flip, ctab, 0, lane);
+    pair_cell<SIGN>(pc[1], A.cg, per, flip, ctab, 1, lane);
+  };
+  Blk<T> s0, s;  // this thread's block of a large level, and of its wave's small level
+
+  // the top level's cells, every global load of a block in flight at once;
+  // the addresses and the reciprocals' tables meanwhile
   {
     const BlkLevel<T> &L = A.L[0];
-    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+    int blk = threadIdx.x;
+    do {
+      const bool in = blk < L.nb;
       int ic, jc, kc;
-      blk_coords(L, blk, ic, jc, kc);
+      blk_coords(L, min(blk, L.nb - 1), ic, jc, kc);
       Two<T> ru[4], rb[4];
 #pragma unroll
       for (int q = 0; q < 4; q++) {
@@ -2457,103 +2573,191 @@ __global__ __launch_bounds__(MAXT) void k_mg_bottom_blocks(BlkArgs<T, TC> args) 
         if (A.zero_top) ru[q] = Two<T>{(T)0, (T)0};
         else ru[q] = *reinterpret_cast<const Two<T> *>(L.u.p + o * L.u.xs + oj * L.u.ys + 2 * kc);
       }
-      T *u = U(0) + blk * BLK, *b = B(0) + blk * BLK;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        u[2 * q] = ru[q].a;
-        u[2 * q + 1] = ru[q].b;
-        b[2 * q] = rb[q].a;
-        b[2 * q + 1] = rb[q].b;
+      if (blk == (int)threadIdx.x) {
+        if (held0) places(s0, 0, blk);
+        if (fs < C && mine(fs)) places(s, fs, lane);
+        for (int l = wave; l < A.nlev; l += nw)
+          if (lane < FACE_CLASSES) {
+            if (l < C) ((Recip<T> *)(smem + A.L[l].toff))[lane] = class_recip<T>(A.L[l].dc, lane);
+            else ((Recip<TC> *)(smem + A.ctoff))[lane] = class_recip<TC>(A.hc, lane);
+          }
       }
-    }
+      if (in) {
+        T *u = U(0) + blk * BLK, *b = B(0) + blk * BLK;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          u[2 * q] = ru[q].a;
+          u[2 * q + 1] = ru[q].b;
+          b[2 * q] = rb[q].a;
+          b[2 * q + 1] = rb[q].b;
+        }
+      }
+      if (held0) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          s0.u[2 * q] = ru[q].a;
+          s0.u[2 * q + 1] = ru[q].b;
+          s0.hb[2 * q] = b_term(L.dc, rb[q].a);
+          s0.hb[2 * q + 1] = b_term(L.dc, rb[q].b);
+        }
+      }
+      blk += blockDim.x;
+    } while (blk < L.nb);
+    __syncthreads();
+    if (held0) recips(s0, 0, threadIdx.x);
   }
-  for (int q = threadIdx.x; q < FACE_CLASSES * A.nlev; q += blockDim.x) {
-    const int l = q / FACE_CLASSES, n = q - l * FACE_CLASSES;
-    if (l < C) ((Recip<T> *)(smem + A.L[l].toff))[n] = class_recip<T>(A.L[l].dc, n);
-    else ((Recip<TC> *)(smem + A.ctoff))[n] = class_recip<TC>(A.hc, n);
-  }
-  __syncthreads();
 
   // down: relax, residual -> the next level's b; the next u starts at zero
-  for (int l = 0; l < C; l++) {
+  auto to_coarse = [&](const Blk<T> &k, int l, int blk) {
     const BlkLevel<T> &L = A.L[l];
-    T *const u = U(l), *const b = B(l);
-    auto to_coarse = [&](const Blk<T> &s, int blk) {
-      int ic, jc, kc;
-      blk_coords(L, blk, ic, jc, kc);
-      const T v = blk_restrict<SIGN>(s, u, b, L.rc);
-      if (l + 1 < C) {
-        const int e = blk_elem(A.L[l + 1], ic, jc, kc);
-        B(l + 1)[e] = v;
-        U(l + 1)[e] = (T)0;
-        A.L[l + 1].b.at(ic, jc, kc) = v;
-      } else {
-        const int e = pair_elem(A.cg, ic, jc, kc);
-        bc[e] = (TC)v;
-        uc[e] = (TC)0;
-        A.cb.at(ic, jc, kc) = v;
-      }
-    };
-    Blk<T> s;
-    if (L.nb <= (int)blockDim.x) {
-      const bool mine = (int)threadIdx.x < L.nb;
-      if (mine) blk_get<SIGN>(s, L, per, flip, u, b, tab(l), threadIdx.x);
-      blk_sweeps<SIGN, true>(s, L, per, flip, u, b, tab(l), A.nu1);
-      if (mine) to_coarse(s, threadIdx.x);
+    int ic, jc, kc;
+    blk_coords(L, blk, ic, jc, kc);
+    const T v = blk_restrict<SIGN>(k, U(l), B(l), L.rc);
+    if (l + 1 < C) {
+      const int e = blk_elem(A.L[l + 1], ic, jc, kc);
+      B(l + 1)[e] = v;
+      U(l + 1)[e] = (T)0;
+      A.L[l + 1].b.at(ic, jc, kc) = v;
     } else {
-      blk_sweeps<SIGN, false>(s, L, per, flip, u, b, tab(l), A.nu1);
+      const int e = pair_elem(A.cg, ic, jc, kc);
+      bc[e] = (TC)v;
+      uc[e] = (TC)0;
+      A.cb.at(ic, jc, kc) = v;
+    }
+  };
+  for (int l = 0; l < fs; l++) {
+    const BlkLevel<T> &L = A.L[l];
+    if (L.nb <= (int)blockDim.x) {
+      const bool in = (int)threadIdx.x < L.nb;
+      if (!held0) set_up(s0, l, threadIdx.x), cells(s0, l);
+      blk_sweeps<SIGN, true>(s0, L, per, flip, U(l), B(l), tab(l), A.nu1);
+      if (in) to_coarse(s0, l, threadIdx.x);
+    } else {
+      blk_sweeps<SIGN, false>(s0, L, per, flip, U(l), B(l), tab(l), A.nu1);
       for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
-        blk_get<SIGN>(s, L, per, flip, u, b, tab(l), blk);
-        to_coarse(s, blk);
+        blk_get<SIGN>(s0, L, per, flip, U(l), B(l), tab(l), blk);
+        to_coarse(s0, l, blk);
       }
     }
     __syncthreads();
   }
-
-  pair_solve<SIGN>(uc, bc, A.cg, A.hc, per, flip, ctab, A.coarse_iters, 0, A.pow2);
-  pair_store<SIGN>(A.cu, uc, A.cg, per, flip);
-
-  // up: prolongation, relax, and the finished level to global memory
-  for (int l = C - 1; l >= 0; l--) {
-    const BlkLevel<T> &L = A.L[l];
-    T *const u = U(l), *const b = B(l);
-    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
-      int ic, jc, kc;
-      blk_coords(L, blk, ic, jc, kc);
-      T v[3][3][3], w[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) w[e] = u[blk * BLK + e];
-      if (l + 1 < C) {
-        const BlkLevel<T> &N = A.L[l + 1];
-        const T *const un = U(l + 1);
-        coarse_around<SIGN>(v, ic, jc, kc, L.bx, L.by, L.bz, per, flip,
-                            [&](int i, int j, int k) { return un[blk_elem(N, i, j, k)]; });
-      } else {
-        coarse_around<SIGN>(v, ic, jc, kc, L.bx, L.by, L.bz, per, flip,
-                            [&](int i, int j, int k) { return (T)uc[pair_elem(A.cg, i, j, k)]; });
+  {
+    PairCell<TC> pc[2];  // the coarsest's cells
+    const bool pairs = nw > 1 && A.cg.n <= 64, early = fs < C;
+    for (int l = fs; l < C; l++) {
+      if (mine(l)) {
+        if (l == fs) recips(s, l, lane);
+        const bool in = lane < A.L[l].nb;
+        cells(s, l);
+        blk_wave<SIGN>(s, in, U(l), A.L[l].dc, A.nu1);
+        if (in) to_coarse(s, l, lane);
+      } else {  // the next level's wave sets itself up meanwhile
+        if (l + 1 < C && mine(l + 1)) set_up(s, l + 1, lane);
+        if (l + 1 == C && pairs && mine(C)) set_up_pairs(pc);
       }
-      blk_prolong(w, v);
+      __syncthreads();
+    }
+    if (pairs) {
+      if (mine(C)) {
+        if (!early) set_up_pairs(pc);
 #pragma unroll
-      for (int e = 0; e < 8; e++) u[blk * BLK + e] = w[e];
-    }
-    __syncthreads();
-    Blk<T> s;
-    if (L.nb <= (int)blockDim.x) {
-      if ((int)threadIdx.x < L.nb) blk_get<SIGN>(s, L, per, flip, u, b, tab(l), threadIdx.x);
-      blk_sweeps<SIGN, true>(s, L, per, flip, u, b, tab(l), A.nu2);
+        for (int n = 0; n < 2; n++)
+          pc[n].u = uc[pc[n].own], pc[n].hb = -A.hc.h * A.hc.h * bc[pc[n].own];
+        if (sizeof(TC) == 4 && A.pow2) pair_wave<SIGN, true>(pc, uc, A.hc, A.coarse_iters, 0);
+        else pair_wave<SIGN, false>(pc, uc, A.hc, A.coarse_iters, 0);
+      }
+      __syncthreads();
     } else {
-      blk_sweeps<SIGN, false>(s, L, per, flip, u, b, tab(l), A.nu2);
+      pair_solve<SIGN>(uc, bc, A.cg, A.hc, per, flip, ctab, A.coarse_iters, 0, A.pow2);
     }
-    for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+  }
+
+  // a finished level to global memory, by the threads id of cnt
+  auto store = [&](int l, int id, int cnt) {
+    if (l == C) {
+      pair_store<SIGN>(A.cu, uc, A.cg, per, flip, id, cnt);
+      return;
+    }
+    const BlkLevel<T> &L = A.L[l];
+    const T *const u = U(l);
+    for (int blk = id; blk < L.nb; blk += cnt) {
       int ic, jc, kc;
       blk_coords(L, blk, ic, jc, kc);
+      T *const o = L.u.p + (int64_t)(2 * ic) * L.u.xs + (2 * jc) * L.u.ys + 2 * kc;
 #pragma unroll
       for (int q = 0; q < 4; q++)
-        *reinterpret_cast<Two<T> *>(L.u.p + (int64_t)(2 * ic + (q >> 1)) * L.u.xs + (2 * jc + (q & 1)) * L.u.ys +
-                                    2 * kc) = Two<T>{u[blk * BLK + 2 * q], u[blk * BLK + 2 * q + 1]};
+        *reinterpret_cast<Two<T> *>(o + (q >> 1) * L.u.xs + (q & 1) * L.u.ys) =
+            Two<T>{u[blk * BLK + 2 * q], u[blk * BLK + 2 * q + 1]};
     }
-    shell_store<SIGN>(L.u, L.mpy, L.mz, per, flip, [&](int i, int j, int k) { return u[blk_elem(L, i, j, k)]; });
+    shell_store<SIGN>(L.u, L.mpy, L.mz, per, flip, id, cnt,
+                      [&](int i, int j, int k) { return u[blk_elem(L, i, j, k)]; });
+  };
+
+  // up: prolongation and relaxation; a finished level is stored by the waves
+  // that the next one leaves idle
+  auto coarse = [&](int l, auto body) {
+    if (l + 1 < C) {
+      const BlkLevel<T> &N = A.L[l + 1];
+      const T *const un = U(l + 1);
+      body([&](int i, int j, int k) { return un[blk_elem(N, i, j, k)]; });
+    } else {
+      body([&](int i, int j, int k) { return (T)uc[pair_elem(A.cg, i, j, k)]; });
+    }
+  };
+  {
+    for (int l = C - 1; l >= fs; l--) {
+      const BlkLevel<T> &L = A.L[l];
+      T *const u = U(l);
+      // a thread per cell, the 8 cells of a block side by side
+      coarse(l, [&](auto at) {
+        for (int t = threadIdx.x; t < 8 * L.nb; t += blockDim.x) {
+          const int blk = t >> 3, e = t & 7;
+          int ic, jc, kc;
+          blk_coords(L, blk, ic, jc, kc);
+          u[blk * BLK + e] = child_prolong<SIGN>(u[blk * BLK + e], e, ic, jc, kc, L.bx, L.by, L.bz, per, flip, at);
+        }
+      });
+      if (mine(l) && l == C - 1) set_up(s, l, lane);
+      __syncthreads();
+      if (mine(l)) {
+        const bool in = lane < L.nb;
+        cells(s, l);
+        blk_wave<SIGN>(s, in, u, L.dc, A.nu2);
+      } else {
+        if (l - 1 >= fs && mine(l - 1)) set_up(s, l - 1, lane);
+        store(l + 1, (wave - (wave > l % nw)) * 64 + lane, (nw - 1) * 64);
+      }
+      __syncthreads();
+    }
   }
+  for (int l = fs - 1; l >= 0; l--) {
+    const BlkLevel<T> &L = A.L[l];
+    T *const u = U(l), *const b = B(l);
+    coarse(l, [&](auto at) {
+      for (int blk = threadIdx.x; blk < L.nb; blk += blockDim.x) {
+        int ic, jc, kc;
+        blk_coords(L, blk, ic, jc, kc);
+        T v[3][3][3], w[8];
+        coarse_around<SIGN>(v, ic, jc, kc, L.bx, L.by, L.bz, per, flip, at);
+#pragma unroll
+        for (int e = 0; e < 8; e++) w[e] = u[blk * BLK + e];
+        blk_prolong(w, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) u[blk * BLK + e] = w[e];
+      }
+    });
+    if (L.nb <= (int)blockDim.x) {
+      if (!held0) set_up(s0, l, threadIdx.x);
+      __syncthreads();
+      cells(s0, l);
+      blk_sweeps<SIGN, true>(s0, L, per, flip, u, b, tab(l), A.nu2);
+    } else {
+      __syncthreads();
+      blk_sweeps<SIGN, false>(s0, L, per, flip, u, b, tab(l), A.nu2);
+    }
+    store(l + 1, threadIdx.x, blockDim.x);
+  }
+  store(0, threadIdx.x, blockDim.x);
 }
 
 // ocu_mg_coarse_relax on pairs: a level by itself, any sizes
@@ -2580,7 +2784,7 @@ __global__ __launch_bounds__(BOT_THREADS) void k_coarse_pairs(PairArgs<TS, TC> A
   for (int q = threadIdx.x; q < FACE_CLASSES; q += blockDim.x) tab[q] = class_recip<TC>(A.c, q);
   __syncthreads();
   pair_solve<SIGN>(uc, bc, A.g, A.c, A.per, A.flip, tab, A.iterations, A.order, A.pow2);
-  pair_store<SIGN>(A.u, uc, A.g, A.per, A.flip);
+  pair_store<SIGN>(A.u, uc, A.g, A.per, A.flip, threadIdx.x, blockDim.x);
 }
 
 // ------------------------------------------------------------------------
@@ -3390,9 +3594,9 @@ int launch_bottom(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_p
     // a thread per block of the top level and per pair of the coarsest
     const int items = std::max(K.L[0].nb, K.cg.n);
     const int threads = std::min(BOT_THREADS, (items + 63) / 64 * 64);
-    // half the threads may hold twice the registers: an FP64 block takes 164
-    // (up to 16^3), and spills 74 of them beyond 512 blocks (45 us against
-    // k_mg_bottom's 105 at 20x20x16 all the same)
+    // half the threads may hold twice the registers: keeping the top level's
+    // block and setting up a small level ahead take 253 in FP64 (without them
+    // 119, which is what 1024 threads leave; 20x20x16 FP64 105 -> 38 us)
     auto kern = threads <= BOT_THREADS / 2
                     ? (K.flip ? k_mg_bottom_blocks<T, TC, true, BOT_THREADS / 2> : k_mg_bottom_blocks<T, TC, false, BOT_THREADS / 2>)
                     : (K.flip ? k_mg_bottom_blocks<T, TC, true, BOT_THREADS> : k_mg_bottom_blocks<T, TC, false, BOT_THREADS>);

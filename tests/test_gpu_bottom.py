@@ -88,6 +88,10 @@ SHAPES = {
     "thin": ((4, 32, 4), 2),
     "wide": ((20, 20, 16), 2),          # 800 blocks: more than half a full workgroup
     "reloaded": ((24, 20, 28), 2),      # 1680 blocks: more than threads
+    "one_wave_deep": ((8, 8, 8), 3),    # one wave for every level
+    "two_waves": ((8, 8, 16), 3),       # a wave per small level, the coarsest back on the first
+    "part_waves": ((12, 8, 24), 3),     # 288 blocks, 36 blocks, coarsest 3 x 2 x 6
+    "four_levels": ((16, 16, 16), 4),
     "long_pairs": ((2, 2, 2052), 2),    # coarsest 1 x 1 x 1026
 }
 
