@@ -23,7 +23,8 @@ __device__ __forceinline__ T interp(int scheme, T u, T x0, T x1) {
 
 // Reading an array around one cell: A(o) is the element at offset o from the
 // cell (o = di*xs + dj*ys + dk in the strides the caller passes).  GAt reads
-// global memory; the marching NS step passes accessors over its LDS window.
+// global memory; the marching NS step passes accessors over its registers and
+// LDS planes.
 template <typename T>
 struct GAt {
   const T *__restrict__ p;  // the cell

@@ -1,4 +1,5 @@
-// The explicit part of one Eqn_IncompressibleNS3D step in one launch.
+// The explicit part of one Eqn_IncompressibleNS3D step in two launches: T's
+// interior, then everything else.
 //
 // The reference's step (eqn_incompressns3d.cu:331-393) runs self-advection,
 // three momentum Laplacians, the thermal force, passive advection of T and
