@@ -167,12 +167,13 @@ class AdvectProjectProblem:
             t.where(m, x.detach().to(g.tensor.dtype), t.zeros((), dtype=g.tensor.dtype), out=g.tensor)
         self._project(self.proj)
         # a state is written where it is kept: the checkpoints, and the last
-        # one in phi; those between alternate between phi and a backward buffer
+        # one in phi; those between alternate between phi and seed, which is
+        # set after them
         last = self.ck[0] if self.steps else self.phi
         D.grid_copy(last, self.phi0)
         for n in range(1, self.steps + 1):
             even = (self.steps - n) % 2 == 0
-            dst = self.ck[n // self.ce] if n % self.ce == 0 and n < self.steps else self.phi if even else self.lam2
+            dst = self.ck[n // self.ce] if n % self.ce == 0 and n < self.steps else self.phi if even else self.seed
             self._step(last, dst)
             last = dst
         self.seed.tensor.zero_()
@@ -200,7 +201,8 @@ class AdvectProjectProblem:
                 self._step(seg[m - 1], seg[m])
             for n in reversed(range(n0, n1)):
                 # the fill's adjoint follows each step (lam's ghosts stay
-                # zero), so the last one is that of phi0's fill
+                # zero: lam and lam2 hold nothing but adjoints), so the last
+                # one is that of phi0's fill
                 D.passive_advect_adjoint_step(self.u, self.v, self.w, seg[n - n0], lam, lam2, self.au, self.av,
                                               self.aw, self.dt, *self.h, self.scheme, self.phi_bc)
                 lam, lam2 = lam2, lam

@@ -216,3 +216,24 @@ def test_two_losses_on_one_problem_are_refused(gpu):
     l2 = A().advect_project_loss(*[2 * x for x in v], p)
     with pytest.raises(RuntimeError, match="ran forward again"):
         (l1 + l2).backward()
+
+
+@pytest.mark.parametrize("steps,ce", [(6, 5), (7, 3), (4, 4)])
+def test_adjoint_steps_get_zero_ghosts(gpu, monkeypatch, steps, ce):
+    """the adjoint step asks for a zero ghost layer of lam: no forward state
+    may be left in a buffer that becomes lam, on a first or repeated pass"""
+    from opencurrent_amd import device as D
+    p = problem(n=(16, 16, 16), steps=steps, ce=ce, bcs=walls("benard"))
+    step, seen = D.passive_advect_adjoint_step, []
+
+    def checked(u, v, w, phi, lam, *rest):
+        d, a = lam.desc, lam.to_host().full().copy()
+        a[d.gx:d.gx + d.nx, d.gy:d.gy + d.ny, d.gz:d.gz + d.nz] = 0
+        seen.append(float(np.abs(a[:d.nx + 2 * d.gx, :d.ny + 2 * d.gy, :d.nz + 2 * d.gz]).max()))
+        step(u, v, w, phi, lam, *rest)
+
+    monkeypatch.setattr(D, "passive_advect_adjoint_step", checked)
+    for _ in range(2):
+        p.forward(*velocity(p))
+        p.backward()
+    assert len(seen) == 2 * steps and max(seen) == 0, seen
