@@ -306,14 +306,18 @@ int ocu_mg_smooth2_ok(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu
  * relax(nu2); every level's u (with ghosts) and b (below the top) is written
  * back.  Arrays u[l], b[l], p[l] and h[3l..3l+2] (hx,hy,hz) describe level
  * top+l; zero_top: the top level's u is the zero grid (not read; needs
- * homogeneous faces).  u[0]'s ghost layer holds its level-1 fill, as it does
- * wherever the solver calls this: with homogeneous faces it is taken from
- * the cells and not read.  Faces must be Neumann or Dirichlet, or periodic
+ * homogeneous faces).  Faces must be Neumann or Dirichlet, or periodic
  * pairs with even counts; the boxes must fit ocu_mg_bottom_lds_bytes() <=
  * ocu_mg_bottom_lds_max(). */
 int ocu_mg_bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p,
                          const double *h, int nlev, const ocu_bc_set *bc, int nu1, int nu2,
                          int coarse_iters, int coarse_mode, int zero_top, void *stream);
+/* The same for a u[0] whose ghost layer is the level-1 fill of its cells, as
+ * it is wherever the solver calls this: the kernel may take the ghosts from
+ * the cells instead of reading them (faster, the same bits) */
+int ocu_mg_bottom_vcycle_filled(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p,
+                                const double *h, int nlev, const ocu_bc_set *bc, int nu1, int nu2,
+                                int coarse_iters, int coarse_mode, int zero_top, void *stream);
 /* LDS bytes a bottom launch over these levels needs (0: invalid request) */
 size_t ocu_mg_bottom_lds_bytes(const ocu_grid3d *u, int nlev, int coarse_mode);
 /* LDS bytes one bottom (or coarse-relax) workgroup may use: 160 KiB */

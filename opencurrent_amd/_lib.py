@@ -106,6 +106,7 @@ HIP_SIGS = {
     "ocu_mg_smooth2": (I, [GP, GP, GP, GP, GP, MP, BP, I, DP, P]),
     "ocu_mg_smooth2_ok": (I, [GP, GP, GP, BP]),
     "ocu_mg_bottom_vcycle": (I, [GP, GP, MP, DP, I, BP, I, I, I, I, I, P]),
+    "ocu_mg_bottom_vcycle_filled": (I, [GP, GP, MP, DP, I, BP, I, I, I, I, I, P]),
     "ocu_mg_bottom_lds_bytes": (C.c_size_t, [GP, I, I]),
     "ocu_mg_bottom_lds_max": (C.c_size_t, []),
     "ocu_mg_coarse_relax": (I, [GP, GP, I, I, MP, BP, D, D, D, I, P]),

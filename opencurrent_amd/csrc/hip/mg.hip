@@ -1960,11 +1960,11 @@ __global__ __launch_bounds__(BOT_THREADS) void k_mg_bottom(BotArgs<T, TC> args) 
 // the bottom of a V-cycle, a thread per coarse cell
 // ------------------------------------------------------------------------
 //
-// The same work as k_mg_bottom (which keeps the rest: inhomogeneous faces,
-// levels that are not exactly halved, unaligned rows) for the hierarchies
-// the solvers make: every
-// level exactly twice the next one, homogeneous faces, and u's ghost layer
-// the level-1 fill of u.  One workgroup on one CU is bound by its issue slots
+// The same work as k_mg_bottom (which keeps the rest: ghosts that are not
+// the fill of u, inhomogeneous faces, levels that are not exactly halved,
+// unaligned rows) for the hierarchies the solvers make: every level exactly
+// twice the next one, homogeneous faces, and u's ghost layer the level-1
+// fill of u.  One workgroup on one CU is bound by its issue slots
 // (16^3: 2048 cells per colour on four SIMDs) and, on the small levels, by
 // the latency of one cell's chain; so:
 //   - a thread owns a block of 2x2x2 cells, the children of one coarse cell.
@@ -3534,7 +3534,7 @@ PairGeom pair_geom(const ocu_grid3d *u) {
 
 // Blocks when every level is exactly twice the next, faces are homogeneous
 // and cell pairs can be loaded as vectors; any other hierarchy that the
-// entry point accepts runs on k_mg_bottom.  Returns the LDS bytes, or 0.
+// entry points accept runs on k_mg_bottom.  Returns the LDS bytes, or 0.
 template <typename T, typename TC>
 size_t blocks_layout(const ocu_grid3d *u, const ocu_grid3d *b, int nlev, const ocu_bc_set *bc, BlkArgs<T, TC> &A) {
   const int C = nlev - 1;
@@ -3571,10 +3571,12 @@ size_t blocks_layout(const ocu_grid3d *u, const ocu_grid3d *b, int nlev, const o
 
 template <typename T, typename TC, int MODE>
 int launch_bottom(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p, const double *h, int nlev,
-                  const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters, int zero_top, hipStream_t stream) {
+                  const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters, int zero_top, bool filled,
+                  hipStream_t stream) {
   BlkArgs<T, TC> K;
   memset(&K, 0, sizeof(K));
-  const size_t blk_bytes = blocks_layout(u, b, nlev, bc, K);
+  // (the blocks take u's ghosts from its cells)
+  const size_t blk_bytes = filled || zero_top ? blocks_layout(u, b, nlev, bc, K) : 0;
   if (blk_bytes && blk_bytes <= BOT_LDS_MAX) {
     for (int l = 0; l + 1 < nlev; l++) {
       K.L[l].dc = dev_c<T>(&p[l]);
@@ -3764,9 +3766,9 @@ size_t ocu_mg_bottom_lds_bytes(const ocu_grid3d *u, int nlev, int coarse_mode) {
                           : bottom_layout<float, float>(u, nlev, 0, (BotArgs<float, float> *)nullptr);
 }
 
-int ocu_mg_bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p, const double *h,
+static int bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p, const double *h,
                          int nlev, const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters, int coarse_mode,
-                         int zero_top, void *stream) {
+                         int zero_top, bool filled, void *stream) {
   const char *what = "ocu_mg_bottom_vcycle";
   OCU_REQUIRE(u && b && p && h && bc, "%s: null argument", what);
   OCU_REQUIRE(nlev >= 2 && nlev <= BOT_MAX, "%s: %d levels (2..%d)", what, nlev, BOT_MAX);
@@ -3801,12 +3803,23 @@ int ocu_mg_bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_
   const size_t bytes = ocu_mg_bottom_lds_bytes(u, nlev, coarse_mode);
   OCU_REQUIRE(bytes > 0 && bytes <= BOT_LDS_MAX, "%s: %zu bytes of LDS exceed %zu", what, bytes, BOT_LDS_MAX);
   if (u[0].dtype == OCU_F64)
-    return launch_bottom<double, double, 0>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, S(stream));
+    return launch_bottom<double, double, 0>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, filled, S(stream));
   if (coarse_mode == 1)
-    return launch_bottom<float, double, 1>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, S(stream));
-  return launch_bottom<float, float, 0>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, S(stream));
+    return launch_bottom<float, double, 1>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, filled, S(stream));
+  return launch_bottom<float, float, 0>(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, zero_top, filled, S(stream));
 }
 
+int ocu_mg_bottom_vcycle(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p, const double *h,
+                         int nlev, const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters, int coarse_mode,
+                         int zero_top, void *stream) {
+  return bottom_vcycle(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, coarse_mode, zero_top, false, stream);
+}
+
+int ocu_mg_bottom_vcycle_filled(const ocu_grid3d *u, const ocu_grid3d *b, const ocu_mg_level_params *p,
+                                const double *h, int nlev, const ocu_bc_set *bc, int nu1, int nu2, int coarse_iters,
+                                int coarse_mode, int zero_top, void *stream) {
+  return bottom_vcycle(u, b, p, h, nlev, bc, nu1, nu2, coarse_iters, coarse_mode, zero_top, true, stream);
+}
 
 int ocu_mg_relax(const ocu_grid3d *u, const ocu_grid3d *b, int color, const ocu_mg_level_params *p,
                  int variant, void *stream) {

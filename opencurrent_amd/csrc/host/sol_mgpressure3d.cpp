@@ -531,8 +531,8 @@ void Sol_MultigridPressure3DDevice<T>::bottom_vcycle(int top) {
   }
   ocu_bc_set cbc = to_c_bc(get_bc_at_level(top));
   int coarse_iters = max3(nx(C) * ny(C), ny(C) * nz(C), nx(C) * nz(C)) / 2;
-  ok_status(ocu_mg_bottom_vcycle(u, b, p, h, nlev, &cbc, nu1, nu2, coarse_iters, _coarse_mode, _u_zero[top] ? 1 : 0,
-                                 ThreadManager::get_compute_stream()),
+  ok_status(ocu_mg_bottom_vcycle_filled(u, b, p, h, nlev, &cbc, nu1, nu2, coarse_iters, _coarse_mode,
+                                        _u_zero[top] ? 1 : 0, ThreadManager::get_compute_stream()),
             "Sol_MultigridPressure3DDevice::bottom_vcycle");
   for (int l = top; l <= C; l++) _u_zero[l] = false;
 }

@@ -1,7 +1,7 @@
-"""The block kernel of the V-cycle's bottom and the pair kernel of the
-coarsest level (2x2x2 cells, or a pair of cells, per thread) against the
-oracle's per-level operations, bit for bit: every level's u with its ghosts
-and the b's below the top.  Sizes: one and several waves of blocks, more
+"""The bottom of a V-cycle and the coarsest level, by the general kernels and
+by those that take u's ghosts from its cells (2x2x2 cells, or a pair of
+cells, per thread), against the oracle's per-level operations, bit for bit:
+every level's u with its ghosts and the b's below the top.  Sizes: one and several waves of blocks, more
 blocks or pairs than a workgroup has threads (blocks reloaded per colour), a
 coarsest level with odd sides; copy, sign-changing and periodic faces, the
 anisotropic factors that FP32 keeps in float (powers of two) and others.
@@ -39,10 +39,13 @@ def level(bc, h):
 
 
 def sweep(u, b, p, bc, h, host=False):
-    """one red-black iteration with the fill that the two colours see"""
+    """one red-black iteration with the fill that the two colours see (each
+    colour's ghosts from the cells it updates: off periodic axes the second
+    colour reads only ghosts of its own, which are as they were)"""
     for color in (0, 1):
         O.lib().orc_mg_relax(u.ptr(), b.ptr(), color, C.byref(p), T.RELAX_HOST if host else T.RELAX_DEVICE)
-        O.lib().orc_bc_fill(0, u.ptr(), C.byref(bc), *h)
+        if color or any(getattr(bc, f).type == T.BC_PERIODIC for f in BCSet.FACES):
+            O.lib().orc_bc_fill(0, u.ptr(), C.byref(bc), *h)
 
 
 def coarsest(u, b, p, bc, h, iters, mode):
@@ -119,23 +122,52 @@ def test_bottom_blocks_match_oracle(gpu, shape, kind, aniso, mode):
         ps.append(p)
     us[0].interior()[:] = 2 * uniform(610, n) - 1
     O.lib().orc_bc_fill(0, us[0].ptr(), C.byref(bc), *hs[0])
-    gus, gbs = [DeviceGrid.from_host(x) for x in us], [DeviceGrid.from_host(x) for x in bs]
-    iters = 5
+    print(f"bottom {shape} {kind} {aniso} {mode}", flush=True)
+    match(us, bs, ps, hs, bc, cmode, ["ocu_mg_bottom_vcycle_filled", "ocu_mg_bottom_vcycle"])
+
+
+def match(us, bs, ps, hs, bc, cmode, entries):
+    """each entry point's bottom against the oracle's"""
+    nlev, iters, hip = len(us), 5, _lib.hip()
     desc = lambda v: (T.Grid3DDesc * nlev)(*[x.desc for x in v])  # noqa: E731
-    hip = _lib.hip()
-    du = desc(gus)
-    need = hip.ocu_mg_bottom_lds_bytes(du, nlev, cmode)
+    dev = [[[DeviceGrid.from_host(x) for x in v] for v in (us, bs)] for _ in entries]
+    need = hip.ocu_mg_bottom_lds_bytes(desc(dev[0][0]), nlev, cmode)
     if need > hip.ocu_mg_bottom_lds_max():
         pytest.skip(f"needs {need} bytes of LDS")
-    print(f"bottom {shape} {kind} {aniso} {mode}", flush=True)
-    _lib.check(hip.ocu_mg_bottom_vcycle(du, desc(gbs), (MGLevelParams * nlev)(*ps),
-                                        (C.c_double * (3 * nlev))(*[x for h in hs for x in h]), nlev, C.byref(bc), 2,
-                                        2, iters, cmode, 0, None), "bottom")
+    for entry, (gus, gbs) in zip(entries, dev):
+        _lib.check(getattr(hip, entry)(desc(gus), desc(gbs), (MGLevelParams * nlev)(*ps),
+                                       (C.c_double * (3 * nlev))(*[x for h in hs for x in h]), nlev, C.byref(bc), 2,
+                                       2, iters, cmode, 0, None), "bottom")
     oracle_vcycle(us, bs, ps, hs, bc, 2, iters, cmode)
+    for entry, (gus, gbs) in zip(entries, dev):
+        for l in range(nlev):
+            ghosts_equal(gus[l].to_host(), us[l], f"{entry}: u level {l}")
+            if l:
+                ghosts_equal(gbs[l].to_host(), bs[l], f"{entry}: b level {l}")
+
+
+@pytest.mark.parametrize("mode", ["f64", "f32", "f32_double"])
+@pytest.mark.parametrize("kind", ["closed", "plates", "values"])
+@pytest.mark.parametrize("shape", ["three_levels", "odd_coarsest", "reloaded"])
+def test_bottom_reads_the_ghosts_it_is_given(gpu, shape, kind, mode):
+    """a ghost layer that is not the fill of u's cells is read as it stands
+    (also beside faces with a value, which only the general kernel takes)"""
+    n, nlev = SHAPES[shape]
+    dtype, cmode = (np.float64, 0) if mode == "f64" else (np.float32, int(mode == "f32_double"))
+    bc = faces("closed" if kind == "closed" else "plates")
+    if kind == "values":
+        bc.zneg, bc.yneg = BC(T.BC_DIRICHELET, .75, 0.0), BC(T.BC_NEUMANN, -.5, 0.0)
+    us, bs, ps, hs = [], [], [], []
     for l in range(nlev):
-        ghosts_equal(gus[l].to_host(), us[l], f"u level {l}")
-        if l:
-            ghosts_equal(gbs[l].to_host(), bs[l], f"b level {l}")
+        m, h = tuple(x >> l for x in n), (.125 * 2 ** l,) * 3
+        u, b = HostGrid(*m, dtype=dtype), HostGrid(*m, dtype=dtype)
+        b.interior()[:] = 2 * uniform(620 + l, m) - 1
+        us.append(u), bs.append(b), hs.append(h)
+        p = level(bc, h)
+        p.h = min(h)
+        ps.append(p)
+    us[0].full()[:] = 2 * uniform(630, us[0].full().shape) - 1
+    match(us, bs, ps, hs, bc, cmode, ["ocu_mg_bottom_vcycle"])
 
 
 @pytest.mark.parametrize("mode", ["f64", "f32", "f32_double"])
