@@ -4120,7 +4120,7 @@ int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations
   size_t tsize = (mode == 1 || u->dtype == OCU_F64) ? 8 : 4;
   size_t shmem = 2 * box * tsize;
   FacesS F = faces_s(bc);
-  if (plain_faces(bc, u, 1)) {
+  if (g.nx > 0 && g.ny > 0 && g.nz > 0 && plain_faces(bc, u, 1)) {
     const size_t bytes = FACE_CLASSES * sizeof(Recip<double>) + 4 * (size_t)g.nx * g.ny * ((g.nz + 1) / 2) * tsize;
     if (bytes <= BOT_LDS_MAX) {
       if (mode == 1) return launch_pairs<float, double>(u, b, iterations, order, p, bc, bytes, S(stream));

@@ -2,7 +2,10 @@
 export every entry point their headers declare; the Python layout and the
 C ABI structs agree with the headers."""
 import ctypes as C
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -71,6 +74,22 @@ def test_invalid_arguments_are_rejected_before_any_launch():
     c.base = 16
     assert hip.ocu_mg_residual_restrict(C.byref(g), C.byref(g), None, C.byref(T.layout(3, 4, 4)), 1.0, 1.0, 1.0,
                                         1.0, None, None) == -1
+
+
+@pytest.mark.parametrize("n", [(0, 4, 4), (4, 0, 4), (4, 4, 0)])
+def test_coarse_relax_of_an_empty_grid_returns(n):
+    """no host division by a side: the call comes back (with an error where no
+    GPU is there to launch on)"""
+    code = ("import ctypes as C\n"
+            "from opencurrent_amd import _lib, _types as T\n"
+            "u, b = T.layout(*%r), T.layout(*%r)\n"
+            "u.base, b.base = 4096, 8192\n"
+            "p, bc = T.MGLevelParams(), T.BCSet.uniform(T.BC_NEUMANN)\n"
+            "_lib.hip().ocu_mg_coarse_relax(C.byref(u), C.byref(b), 2, 0, C.byref(p), C.byref(bc), 1., 1., 1., 0, None)\n"
+            "print('returned')\n" % (n, n))
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")  # never a launch on these addresses
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.split()[-1:] == ["returned"], (r.returncode, r.stderr[-300:])
 
 
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
