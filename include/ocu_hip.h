@@ -330,13 +330,17 @@ size_t ocu_mg_bottom_lds_max(void);
  * mode 1: FP32 grids relaxed in double (copy in, `iterations` host-order
  *   RB-GS iterations with a level-1 ghost fill after every colour, round
  *   back to float) - the coarsest solve of the mixed-precision solver.
- * order: 0 red-black, 1 black-red, 2 symmetric (as relax()).  u's ghost layer
- * holds its fill, as it does wherever the solver calls this: with
- * homogeneous faces it is taken from the cells and not read.  A grid beyond
+ * order: 0 red-black, 1 black-red, 2 symmetric (as relax()).  A grid beyond
  * one workgroup's LDS is relaxed in global memory. */
 int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
                         const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy,
                         double hz, int mode, void *stream);
+/* The same for a u whose ghost layer is the level-1 fill of its cells, as it
+ * is wherever the solver calls this: the kernel may take the ghosts from the
+ * cells instead of reading them (faster, the same bits) */
+int ocu_mg_coarse_relax_filled(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
+                               const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy,
+                               double hz, int mode, void *stream);
 
 /* ---------------- mixed-precision iterative refinement -------------------- */
 

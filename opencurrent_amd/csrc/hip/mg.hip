@@ -4100,9 +4100,9 @@ static int coarse_relax_global(const ocu_grid3d *u, const ocu_grid3d *b, CoarseG
   OCU_HIP_LAUNCHED("ocu_mg_coarse_relax");
 }
 
-int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
+static int coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
                         const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy, double hz,
-                        int mode, void *stream) {
+                        int mode, bool filled, void *stream) {
   if (int e = check_pair(u, b, "ocu_mg_coarse_relax")) return e;
   OCU_REQUIRE(p && bc, "ocu_mg_coarse_relax: null params");
   OCU_REQUIRE(order >= 0 && order <= 2, "ocu_mg_coarse_relax: bad order %d", order);
@@ -4120,7 +4120,8 @@ int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations
   size_t tsize = (mode == 1 || u->dtype == OCU_F64) ? 8 : 4;
   size_t shmem = 2 * box * tsize;
   FacesS F = faces_s(bc);
-  if (g.nx > 0 && g.ny > 0 && g.nz > 0 && plain_faces(bc, u, 1)) {
+  // (the pairs take u's ghosts from its cells)
+  if (filled && g.nx > 0 && g.ny > 0 && g.nz > 0 && plain_faces(bc, u, 1)) {
     const size_t bytes = FACE_CLASSES * sizeof(Recip<double>) + 4 * (size_t)g.nx * g.ny * ((g.nz + 1) / 2) * tsize;
     if (bytes <= BOT_LDS_MAX) {
       if (mode == 1) return launch_pairs<float, double>(u, b, iterations, order, p, bc, bytes, S(stream));
@@ -4145,6 +4146,18 @@ int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations
                                                             (float)hx, (float)hy, (float)hz, iterations, order);
   }
   OCU_HIP_LAUNCHED("ocu_mg_coarse_relax");
+}
+
+int ocu_mg_coarse_relax(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
+                        const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy, double hz,
+                        int mode, void *stream) {
+  return coarse_relax(u, b, iterations, order, p, bc, hx, hy, hz, mode, false, stream);
+}
+
+int ocu_mg_coarse_relax_filled(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int order,
+                               const ocu_mg_level_params *p, const ocu_bc_set *bc, double hx, double hy, double hz,
+                               int mode, void *stream) {
+  return coarse_relax(u, b, iterations, order, p, bc, hx, hy, hz, mode, true, stream);
 }
 
 }  // extern "C"

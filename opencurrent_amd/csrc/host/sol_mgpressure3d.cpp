@@ -623,8 +623,8 @@ void Sol_MultigridPressure3DDevice<T>::relax_coarsest(int level, int iterations,
   ocu_grid3d u = get_u(level).desc(), b = get_b(level).desc();
   ocu_bc_set cbc = to_c_bc(get_bc_at_level(level));
   int ord = order == RO_RED_BLACK ? 0 : order == RO_BLACK_RED ? 1 : 2;
-  ok_status(ocu_mg_coarse_relax(&u, &b, iterations, ord, &p, &cbc, hx(level), hy(level), hz(level), _coarse_mode,
-                                ThreadManager::get_compute_stream()),
+  ok_status(ocu_mg_coarse_relax_filled(&u, &b, iterations, ord, &p, &cbc, hx(level), hy(level), hz(level),
+                                       _coarse_mode, ThreadManager::get_compute_stream()),
             "Sol_MultigridPressure3DDevice::relax_on_host");
 }
 

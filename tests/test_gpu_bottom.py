@@ -182,10 +182,17 @@ def test_coarse_pairs_match_oracle(gpu, n, kind, mode, order):
     b.interior()[:] = 2 * uniform(701, n) - 1
     O.lib().orc_bc_fill(0, u.ptr(), C.byref(bc), *h)
     p = O.level_params(bc, 0, *h)
-    gu, gb = DeviceGrid.from_host(u), DeviceGrid.from_host(b)
     print(f"pairs {n} {kind} {mode} {order}", flush=True)
-    _lib.check(_lib.hip().ocu_mg_coarse_relax(gu.ptr(), gb.ptr(), 6, order, C.byref(p), C.byref(bc), *h, cmode, None),
-               "coarse relax")
+    match_coarse(u, b, p, bc, h, order, cmode, ["ocu_mg_coarse_relax_filled", "ocu_mg_coarse_relax"])
+
+
+def match_coarse(u, b, p, bc, h, order, cmode, entries):
+    """each entry point's relaxation against the oracle's"""
+    dev = [[DeviceGrid.from_host(x) for x in (u, b)] for _ in entries]
+    for entry, (gu, gb) in zip(entries, dev):
+        _lib.check(getattr(_lib.hip(), entry)(gu.ptr(), gb.ptr(), 6, order, C.byref(p), C.byref(bc), *h, cmode, None),
+                   "coarse relax")
+    dtype = u.buf.dtype
     work = [HostGrid.congruent(x, dtype=np.float64 if cmode else dtype) for x in (u, b)]
     work[0].buf[:], work[1].buf[:] = u.buf, b.buf
     for it in range(6):
@@ -195,7 +202,22 @@ def test_coarse_pairs_match_oracle(gpu, n, kind, mode, order):
             O.lib().orc_bc_fill(0, work[0].ptr(), C.byref(bc), *h)
     want = u.copy()
     want.buf[:] = work[0].buf.astype(dtype)
-    ghosts_equal(gu.to_host(), want, "u")
+    for entry, (gu, gb) in zip(entries, dev):
+        ghosts_equal(gu.to_host(), want, f"{entry}: u")
+
+
+@pytest.mark.parametrize("mode", ["f64", "f32", "f32_double"])
+@pytest.mark.parametrize("kind", ["closed", "plates", "periodic"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (6, 4, 10), (12, 10, 14)])
+@pytest.mark.parametrize("order", [0, 1, 2])
+def test_coarse_relax_reads_the_ghosts_it_is_given(gpu, n, kind, mode, order):
+    """a ghost layer that is not the fill of u's cells is read as it stands"""
+    dtype, cmode = (np.float64, 0) if mode == "f64" else (np.float32, int(mode == "f32_double"))
+    bc, h = faces(kind), (.5, .5, .5)
+    u, b = HostGrid(*n, dtype=dtype), HostGrid(*n, dtype=dtype)
+    u.full()[:] = 2 * uniform(720, u.full().shape) - 1
+    b.interior()[:] = 2 * uniform(721, n) - 1
+    match_coarse(u, b, O.level_params(bc, 0, *h), bc, h, order, cmode, ["ocu_mg_coarse_relax"])
 
 
 def test_faces_the_blocks_do_not_take(gpu):

@@ -76,8 +76,9 @@ def test_invalid_arguments_are_rejected_before_any_launch():
                                         1.0, None, None) == -1
 
 
+@pytest.mark.parametrize("entry", ["ocu_mg_coarse_relax", "ocu_mg_coarse_relax_filled"])
 @pytest.mark.parametrize("n", [(0, 4, 4), (4, 0, 4), (4, 4, 0)])
-def test_coarse_relax_of_an_empty_grid_returns(n):
+def test_coarse_relax_of_an_empty_grid_returns(n, entry):
     """no host division by a side: the call comes back (with an error where no
     GPU is there to launch on)"""
     code = ("import ctypes as C\n"
@@ -85,8 +86,8 @@ def test_coarse_relax_of_an_empty_grid_returns(n):
             "u, b = T.layout(*%r), T.layout(*%r)\n"
             "u.base, b.base = 4096, 8192\n"
             "p, bc = T.MGLevelParams(), T.BCSet.uniform(T.BC_NEUMANN)\n"
-            "_lib.hip().ocu_mg_coarse_relax(C.byref(u), C.byref(b), 2, 0, C.byref(p), C.byref(bc), 1., 1., 1., 0, None)\n"
-            "print('returned')\n" % (n, n))
+            "_lib.hip().%s(C.byref(u), C.byref(b), 2, 0, C.byref(p), C.byref(bc), 1., 1., 1., 0, None)\n"
+            "print('returned')\n" % (n, n, entry))
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")  # never a launch on these addresses
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.split()[-1:] == ["returned"], (r.returncode, r.stderr[-300:])
