@@ -3659,6 +3659,9 @@ int launch_pairs(const ocu_grid3d *u, const ocu_grid3d *b, int iterations, int o
   OCU_HIP_LAUNCHED("ocu_mg_coarse_relax");
 }
 
+// byte offsets of a grid's cells fit an int, as the tile kernel keeps them
+bool tile_offsets_fit(const ocu_grid3d *g) { return g->allocated < (int64_t)INT_MAX / 8; }
+
 // Two iterations by tiles: every side even (2x2x2 blocks) and two blocks or
 // more, the faces of the block kernels, at least 14 cells along a periodic
 // axis (so that one step wraps the box) and rows that pairs of cells can be
@@ -3671,8 +3674,7 @@ bool smooth_tile_ok(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_g
     if (n[a] % 2 || n[a] < 4 || (per[a] && n[a] < 14)) return false;
   // (the tile's number is decoded by mdiv)
   if ((int64_t)((n[0] + 7) / 8) * ((n[1] + 7) / 8) * ((n[2] + 7) / 8) >= 1 << 15) return false;
-  for (const ocu_grid3d *g : {u_in, b})  // byte offsets of cells fit an int
-    if (g->allocated >= (int64_t)INT_MAX / 8) return false;
+  if (!tile_offsets_fit(u_in) || !tile_offsets_fit(b)) return false;
   return plain_faces(bc, u_in, 1) && row_aligned(u_in, 2) && row_aligned(u_out, 2) && row_aligned(b, 2);
 }
 
@@ -3744,6 +3746,10 @@ int ocu_mg_smooth2(const ocu_grid3d *u_in, const ocu_grid3d *u_out, const ocu_gr
     if (int e = check_grid(g, what)) return e;
     OCU_REQUIRE(g->dtype == u_in->dtype && u_in->nx == 2 * g->nx && u_in->ny == 2 * g->ny && u_in->nz == 2 * g->nz,
                 "%s: the coarse grids must be half of u", what);
+    if (!tile_offsets_fit(g)) {
+      set_error("%s: a coarse grid's allocation is too large for 32-bit offsets", what);
+      return OCU_ERR_UNSUPPORTED;
+    }
   }
   if (!smooth_tile_ok(u_in, u_out, b, bc)) {
     set_error("%s: needs even sides, homogeneous Neumann, Dirichlet or paired periodic faces and aligned rows", what);

@@ -93,6 +93,26 @@ def test_coarse_relax_of_an_empty_grid_returns(n, entry):
     assert r.returncode == 0 and r.stdout.split()[-1:] == ["returned"], (r.returncode, r.stderr[-300:])
 
 
+@pytest.mark.parametrize("which", ["u_coarse", "b_coarse"])
+def test_smooth2_refuses_coarse_grids_beyond_its_offsets(which):
+    """the kernel's byte offsets are 32-bit: a coarse grid padded beyond them
+    is refused (in a process that sees no GPU: never a launch on these
+    addresses)"""
+    code = ("import ctypes as C\n"
+            "from opencurrent_amd import _lib, _types as T\n"
+            "u, o, b = (T.layout(4, 4, 4) for _ in range(3))\n"
+            "wide = T.layout(2, 2, 2, 1, 1, 1, 0, 0, 1 << 25)\n"
+            "for q, g in enumerate((u, o, b, wide)): g.base = 4096 * (q + 1)\n"
+            "p, bc = T.MGLevelParams(), T.BCSet.uniform(T.BC_NEUMANN)\n"
+            "uc, bc_out = (C.byref(wide), None) if %r == 'u_coarse' else (None, C.byref(wide))\n"
+            "_lib.hip().ocu_mg_smooth2(C.byref(u), C.byref(o), C.byref(b), uc, bc_out, C.byref(p), C.byref(bc), 0, None,\n"
+            "                          None)\n"
+            "print(_lib.last_error())\n" % which)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "32-bit offsets" in r.stdout, (r.returncode, r.stdout[-300:], r.stderr[-300:])
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "LIBDIR", tmp_path)
     monkeypatch.setattr(_lib, "_hip", None)
