@@ -258,7 +258,7 @@ __global__ __launch_bounds__(MTK *MJ) void k_ns_march(NSStep<T> s, int tiles_k, 
     const int per_ = f == 3 ? s.tper : s.fper;
     const int jj = wrapped(j0 - R + wj, s.ny, s.ny + (R == 2 && f == 1), R == 2 && (per_ & 2));
     const int kk = wrapped(k0 - R + wk, s.nz, s.nz + (R == 2 && f == 2), R == 2 && (per_ & 4));
-    return (jj + s.gy) * s.pnz + kk + s.gz;
+    return (unsigned)(jj + s.gy) * (unsigned)s.pnz + (unsigned)(kk + s.gz);
   };
   const bool has_halo = tid < W::HALO;
   int hwj, hwk;  // rows above and below the tile, then the row ends
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(MTK *MJ) void k_ns_march(NSStep<T> s, int tiles_k, 
     }
   }
   const int hcell = hwj * W::WK + hwk;
-  int own_e[4], halo_e[4];
+  unsigned own_e[4], halo_e[4];
 #pragma unroll
   for (int f = 0; f < 4; f++) own_e[f] = element(f, ty + R, tx + R), halo_e[f] = element(f, hwj, hwk);
   auto at = [&](int f, int q) {
