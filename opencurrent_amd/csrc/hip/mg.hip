@@ -2683,7 +2683,7 @@ __global__ __launch_bounds__(MAXT) void k_mg_bottom_blocks(BlkArgs<T, TC> args) 
     for (int blk = id; blk < L.nb; blk += cnt) {
       int ic, jc, kc;
       blk_coords(L, blk, ic, jc, kc);
-      T *const o = L.u.p + (int64_t)(2 * ic) * L.u.xs + (2 * jc) * L.u.ys + 2 * kc;
+      T *const o = L.u.p + (int64_t)(2 * ic) * L.u.xs + (int64_t)(2 * jc) * L.u.ys + 2 * kc;
 #pragma unroll
       for (int q = 0; q < 4; q++)
         *reinterpret_cast<Two<T> *>(o + (q >> 1) * L.u.xs + (q & 1) * L.u.ys) =
