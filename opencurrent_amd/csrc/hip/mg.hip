@@ -169,8 +169,11 @@ __device__ __forceinline__ T relax_pt_host(const HostC<T> &c, T uc, T zm, T zp, 
 //   FP64: two fused corrections of x*r.  The first leaves a faithful
 //     quotient, whose remainder is exact, and by Markstein's theorem the
 //     second then rounds correctly, r being the correctly rounded 1/d;
-//     div_fixup gives the special operands their IEEE results.  (|x| below
-//     2^-960 would make the remainder inexact: one unit of a 1e-290 value.)
+//     div_fixup gives the special operands their IEEE results, and infinity
+//     where the quotient overflows (a diagonal below one, which the solvers'
+//     factors never make: the corrections of an infinite x*r are NaN).  (|x|
+//     below 2^-960 would make the remainder inexact: one unit of a 1e-290
+//     value.)
 template <typename T> struct Recip;
 template <> struct Recip<float> {
   double r;
