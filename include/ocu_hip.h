@@ -507,7 +507,7 @@ int ocu_pcg_diag_precond(const ocu_grid3d *dst, const ocu_grid3d *src, const ocu
 int ocu_grid_dot(const ocu_grid3d *a, const ocu_grid3d *b, void *workspace, double *out, void *stream);
 
 /* The explicit part of Eqn_IncompressibleNS3D<T>::advance_one_step
- * (eqn_incompressns3d.cu:331-393) in one launch: self-advection, viscous
+ * (eqn_incompressns3d.cu:331-393) in two launches: self-advection, viscous
  * diffusion and thermal force of u, v, w, passive advection and diffusion
  * of the temperature, the forward-Euler (or Adams-Bashforth) combination
  * linear_combination(1, x, a_dt, dx) [+ linear_combination(1, x, a_ab,

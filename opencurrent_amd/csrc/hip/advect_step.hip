@@ -15,9 +15,10 @@
 //     product of the cell and the face next to it, and the cell it derives
 //     from adds it in bc_adjoint_nocorners' order; ghosts are not stored.
 // Same operations in the same order as the separate launches, bit for bit.
-// Bound by memory (forward 5 grids read and 1 written, adjoint 9 and 4): at
-// 128^3 a step takes 10 us FP32 and 16 FP64 (21.9 FP32 as three launches), an
-// adjoint step 21 and 36 us (41.9 FP32 as two), 5 TB/s.
+// Bound by memory (forward 4 grids read and 1 written, adjoint 8 and 4): at
+// 128^3 a step takes 10 us FP32 and 16 FP64 (4.2 and 5.2 TB/s; 21.9 FP32 as
+// three launches), an adjoint step 21 and 36 us (4.8 and 5.6 TB/s; 41.9 FP32
+// as two).
 #include <algorithm>
 
 #include "advect.h"
@@ -313,7 +314,7 @@ int rows_width(int nz, std::initializer_list<const ocu_grid3d *> grids) {
 
 // chunks of planes, for about 4096 waves.  The forward march reads a plane
 // ahead and loses two planes per chunk (256^3 FP32: 70 us by 16 planes, 93 by
-// one); the adjoint reads 9 grids and writes 4 with nothing ahead, so beyond
+// one); the adjoint reads 8 grids and writes 4 with nothing ahead, so beyond
 // two planes a wave's chain of planes costs more than the plane it keeps
 // (256^3 FP32: 222 us by 16, 186 by two, 184 by one; 128^3 FP32 21 by any).
 void set_chunks(int nx, int ny, int most, int &tiles_j, int &ichunk, int &ntiles) {

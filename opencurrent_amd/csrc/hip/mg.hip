@@ -2380,9 +2380,10 @@ __device__ __forceinline__ void pair_cell(PairCell<T> &s, const PairGeom &g, con
 }
 
 // do_cpu_solve's update with b's term in hand.  P2: T is float and the
-// three factors are powers of two, so a product with one is exact and the
-// float sum of two floats is what rounding their double sum gives (double
-// keeps more than twice float's bits); the sums stay in float then.
+// three factors are powers of two, so a product with one is exact (down to
+// float's denormals) and the float sum of two floats is what rounding their
+// double sum gives (double keeps more than twice float's bits); the sums stay
+// in float then.
 template <bool P2, typename T>
 __device__ __forceinline__ T relax_host_q(const HostC<T> &c, T uc, T zm, T zp, T ym, T yp, T xm, T xp, T hb,
                                           const Recip<T> &q) {

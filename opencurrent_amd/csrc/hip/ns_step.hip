@@ -7,13 +7,14 @@
 // forward-Euler / Adams-Bashforth combinations (linear_combination,
 // grid3ddev.cu:283-349) and the no-corner ghost fill of T, then (AB2) copies
 // the tendencies to the "last" grids: about 38 grid passes of memory traffic
-// per cell.  Here one thread per element of the padded allocation computes
-// every tendency of its cell in registers (the same device functions, in the
-// same order, as the per-operator kernels), combines it with the old value
-// and writes the new u, v, w and T into a second set of buffers (the caller
-// swaps them in afterwards): 4 grids read, 4 written (plus, for AB2, the
-// last tendencies read and this step's written).  Every element of the new
-// buffers receives exactly what the in-place sequence leaves in the old one:
+// per cell.  Here every tendency of a cell is computed in registers (the same
+// device functions, in the same order, as the per-operator kernels), combined
+// with the old value and written with the new u, v, w and T into a second set
+// of buffers (the caller swaps them in afterwards): k_ns_march does T's
+// interior, k_ns_shell the other elements of the padded allocation; 4 grids
+// read, 4 written (plus, for AB2, the last tendencies read and this step's
+// written).  Every element of the new buffers receives exactly what the
+// in-place sequence leaves in the old one:
 //   - cells the combination covers get old*1 + d*a_dt (+ last*a_ab);
 //   - with the reference's whole-allocation combination (allocation waste
 //     <= 3%) the other elements get old*1 + 0*a_dt (+ 0*a_ab), the tendency
@@ -37,7 +38,7 @@ struct NSStep {
   Inv<T> ih, ih2;
   T nu, kappa, tcoef, a_dt, a_ab, th[3];
   Faces tf;
-  int64_t xs, ys, shift, vnbr;
+  int64_t xs, ys, shift;
   int pre, nx, ny, nz, gx, gy, gz, pnx, pny, pnz;
   int scheme, fper, tper, vaxis, flat, keep, use_last, visc, tdiff;
 };
@@ -110,8 +111,8 @@ __device__ __forceinline__ void ns_prepad(const NSStep<T> &s, int64_t e) {
 // thread each, after the pre-padding: the planes outside the interior's x
 // range (count na), then the rows outside its y range (nb), then the row ends
 // (nc).  I: the type of the element count (a thread's divisions take longer
-// than its copies in 64 bits).  Bound by the row ends, 16 elements of each row
-// of eight grids.
+// than its copies in 64 bits).  Bound by the row ends: pnz - nz elements of
+// each row of eight grids.
 template <typename T, typename I>
 __global__ __launch_bounds__(256) void k_ns_shell(NSStep<T> s, I na, I nb, I nc) {
   I q = (I)blockIdx.x * 256 + threadIdx.x;
@@ -418,7 +419,6 @@ int launch_ns_step(const ocu_grid3d *const *in, const ocu_grid3d *const *out, co
   s.xs = (int64_t)g->pny * g->pnz, s.ys = g->pnz, s.shift = g->shift;
   const int vd = p->vertical_direction;
   s.vaxis = (vd & OCU_DIR_XAXIS_FLAG) ? 0 : (vd & OCU_DIR_YAXIS_FLAG) ? 1 : 2;
-  s.vnbr = s.vaxis == 0 ? s.xs : s.vaxis == 1 ? s.ys : 1;
   s.pre = (int)(g->shift - ((int64_t)g->gx * g->pny * g->pnz + (int64_t)g->gy * g->pnz + g->gz));
   s.nx = p->nx, s.ny = p->ny, s.nz = p->nz, s.gx = g->gx, s.gy = g->gy, s.gz = g->gz;
   s.pnx = g->pnx, s.pny = g->pny, s.pnz = g->pnz;

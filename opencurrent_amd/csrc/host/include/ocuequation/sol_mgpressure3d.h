@@ -177,7 +177,6 @@ class Sol_MultigridPressure3DDevice : public Sol_MultigridPressure3DBase {
   bool defer_ok(int level);
   void materialize(int level);
   void run_prolong(int coarse_level, int fine_level);
-  // level l is about to change: a pending prolongation that reads it runs first
   // the launch by tiles is the faster one at this level
   bool tile_ok(int level);
   void run_tile(int level, int coarse_level, bool norms);
@@ -185,6 +184,7 @@ class Sol_MultigridPressure3DDevice : public Sol_MultigridPressure3DBase {
   bool prolong_sweep_ok(int level);
   char level_state(int l) const;
   void set_level_state(int l, char s);
+  // level l is about to change: a pending prolongation that reads it runs first
   void flush_reader(int level) {
     if (level >= 1 && _u_pro[level - 1]) materialize(level - 1);
   }

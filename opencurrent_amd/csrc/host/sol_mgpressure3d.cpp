@@ -430,7 +430,8 @@ bool Sol_MultigridPressure3DDevice<T>::defer_ok(int level) {
 // (16.3 -> 8.0), 64^3 17.4 -> 9.4 (19.1 -> 10.4), 96x80x112 24.6 -> 24.8
 // (28.2 -> 26.1), 128^3 37.0 -> 51.8.  So up to 2^20 cells in FP32 and 3/4 of
 // that in FP64.  Where the fused sweep does not run (periodic z, 13 us a
-// colour at 128^3 in FP32) the tiles are the faster ones at any size they take.
+// colour at 128^3 in FP32) the tiles are the faster ones at any size they take
+// (below 2^15 tiles of 8^3: a periodic 256^3 level runs one colour a launch).
 template <typename T>
 bool Sol_MultigridPressure3DDevice<T>::tile_ok(int level) {
   if (!use_fused_relax || store_residuals || level >= _num_levels - 1) return false;
@@ -782,8 +783,9 @@ void Sol_MultigridPressure3DDevice<T>::norms_read(int fine_level, double *l2, do
 }
 
 // what a segment's launches depend on besides the grids (fixed from
-// initialize_storage on): options, faces, the stream, and the deferred
-// clears and prolongations of every level
+// initialize_storage on): options, faces, the stream, and per level the
+// deferred clear, prolongation and relaxation and which of its two buffers
+// holds u
 template <typename T>
 std::vector<long long> Sol_MultigridPressure3DDevice<T>::segment_key(void *stream) const {
   std::vector<long long> k = {nu1, nu2, use_fused_relax, use_bottom, use_fused_prolong, store_residuals,
