@@ -233,7 +233,8 @@ __global__ void k_mac_z(DGrid<T> u, DGrid<T> v, DGrid<T> w, Faces f, int nx, int
 // a place's value is another place's, a multiple of it or a face's value, and
 // where that ends no pass writes, so nothing is read that this launch writes;
 // places that two passes write get the same value twice.  128^3 FP64 11.1 us as
-// three launches, 6.3 as one; 96x64x48 FP32 10.2, 6.5.
+// three launches, 6.3 as one; 96x64x48 FP32 10.2, 6.5; 512x512x256 FP64 119, 99
+// (the z faces' single elements).
 template <typename T>
 struct MacFill {
   DGrid<T> a[3];         // u, v, w
